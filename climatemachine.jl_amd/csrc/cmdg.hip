@@ -89,7 +89,8 @@ struct cmdg_ctx {
     AffArrays AA{};
     double *d_geo = nullptr, *d_W = nullptr, *d_Wf = nullptr;
     int32_t *d_nbe = nullptr;
-    double *d_f2tr = nullptr, *d_str = nullptr;  // face traces
+    double *d_nu = nullptr;    // FP64 path: viscosity planes (Smagorinsky-Lilly)
+    double *d_str = nullptr;   // static face trace
     int32_t *d_cls = nullptr;  // static-field class of each element (null: none)
     double *d_sa = nullptr;    // static fields by class
     int32_t *d_order = nullptr;  // tiled traversal order of the affine launches (null: none)
@@ -175,7 +176,7 @@ int launch_gradient_impl(cmdg_ctx *c, const double *Q, double *Qcopy, int write_
                        Q, c->d_aux, c->d_gf32, write_aux, c->d_mlp)
 #define CMDG_GRAD_AFF(SMAG, BUOY)                                                                               \
     hipLaunchKernelGGL((k_gradient_aff<Nq, SMAG, BUOY>), grid, block, 0, c->stream, c->P, c->AA, ES, Q, c->d_aux, \
-                       c->d_gf, c->d_f2tr, write_aux)
+                       c->d_gf, c->d_nu, write_aux)
     if (c->mixed) {
         if (c->learned) {
             if (buoy) CMDG_GRAD_MIX(true, true, true);
@@ -209,16 +210,18 @@ int launch_tendency_impl(cmdg_ctx *c, const double *Q, double *tend, double alph
 #define CMDG_TEND_MIX(DIFF, ISO, MODE)                                                                           \
     hipLaunchKernelGGL((k_tendency_mix<Nq, DIFF, ISO, MODE>), grid, block, 0, c->stream, c->P, c->MP, c->AA, ES, Q, \
                        c->d_gf32, c->d_aux, tend, alpha, beta, Qout, rka, bdt, write_aux, dq_store)
+#define CMDG_TEND_AFF(DIFF, NNU, MODE)                                                                            \
+    hipLaunchKernelGGL((k_tendency_aff<Nq, DIFF, NNU, MODE>), grid, block, 0, c->stream, c->P, c->AA, ES, Q,      \
+                       c->d_gf, c->d_nu, c->d_aux, tend, alpha, beta, Qout, rka, bdt, write_aux, dq_store)
 #define CMDG_TEND(DIFF, SMAG, MODE)                                                                               \
     do {                                                                                                          \
         if (c->mixed) {                                                                                           \
             if (!DIFF || c->iso32) CMDG_TEND_MIX(DIFF, true, MODE);                                               \
             else CMDG_TEND_MIX(DIFF, false, MODE);                                                                \
-        } else if (c->affine)                                                                                     \
-            hipLaunchKernelGGL((k_tendency_aff<Nq, DIFF, SMAG, MODE>), grid, block, 0, c->stream, c->P, c->AA,    \
-                               ES, Q, c->d_gf, c->d_f2tr, c->d_aux, tend, alpha, beta, Qout, rka, bdt,      \
-                               write_aux, dq_store);                                                              \
-        else                                                                                                      \
+        } else if (c->affine) {                                                                                   \
+            if (c->P.a_gPhi >= 0) CMDG_TEND_AFF(DIFF, viscosity_planes(SMAG, true), MODE);                        \
+            else CMDG_TEND_AFF(DIFF, viscosity_planes(SMAG, false), MODE);                                        \
+        } else                                                                                                    \
             hipLaunchKernelGGL((k_tendency<Nq, DIFF, SMAG, MODE>), grid, block, 0, c->stream, c->P, c->A, Q,      \
                                c->d_gf, c->d_aux, tend, alpha, beta, Qout, rka, bdt, write_aux, dq_store);       \
     } while (0)
@@ -233,6 +236,7 @@ int launch_tendency_impl(cmdg_ctx *c, const double *Q, double *tend, double alph
     }
 #undef CMDG_TEND
 #undef CMDG_TEND_MIX
+#undef CMDG_TEND_AFF
     return check_hip(c, hipGetLastError(), "tendency launch");
 }
 
@@ -707,9 +711,10 @@ int create_impl(const cmdg_desc *d, const cmdg_brick *brick, void *stream, cmdg_
             const char *tenv = std::getenv("CMDG_NEIGHBOUR_STATIC_TRACE");  // 1: always read it
             c->AA.aux_cont = (cont && !(tenv && tenv[0] == '1')) ? 1 : 0;
             if ((rc = upload(c, &c->d_str, st.data(), st.size()))) return rc;
-            // the FP64 second-order face trace (mixed contexts carry the stress form instead)
-            if (d->precision != CMDG_MIXED && c->diffusive &&
-                (rc = upload<double>(c, &c->d_f2tr, nullptr, (size_t)E * 6 * TR_F2 * Nfp)))
+            // the FP64 viscosity planes (mixed contexts carry the stress form instead)
+            const int nnu = viscosity_planes(c->smag, P.a_gPhi >= 0);
+            if (d->precision != CMDG_MIXED && nnu > 0 &&
+                (rc = upload<double>(c, &c->d_nu, nullptr, (size_t)Np * nnu * E)))
                 return rc;
             c->AA.geo = c->d_geo;
             c->AA.nbe = c->d_nbe;
@@ -877,7 +882,7 @@ int cmdg_destroy(cmdg_ctx *c) {
     (void)hipFree(c->d_nbe);
     (void)hipFree(c->d_W);
     (void)hipFree(c->d_Wf);
-    (void)hipFree(c->d_f2tr);
+    (void)hipFree(c->d_nu);
     (void)hipFree(c->d_str);
     (void)hipFree(c->d_cls);
     (void)hipFree(c->d_sa);

@@ -9,13 +9,12 @@
 // component of the general formula is dropped; for finite data this changes no
 // result bit.
 //
-// A face reads its neighbour's state straight from the neighbour's volume state
-// (25 values per face and variable; the kernels that update the state write it to
-// another buffer than the one they read).  Derived neighbour data reaches a face
-// through face traces: face-major arrays (nelem, 6, nvar, Nfp) in which the 25
-// values a neighbour needs for one face and one variable are contiguous -- the
-// second-order flux rows, written by the gradient kernel, and the static fields
-// (Phi, p_ref), written once at set-up.
+// A face reads its neighbour's state and gradient flux straight from the neighbour's
+// volume (25 values per face and variable; the kernels that update the state write it to
+// another buffer than the one they read).  The static fields (Phi, p_ref), where the two
+// sides differ, reach a face through a face trace written once at set-up: a face-major
+// array (nelem, 6, nvar, Nfp) in which the 25 values a neighbour needs for one face and
+// one variable are contiguous.
 #pragma once
 #include "cmdg_physics.h"
 
@@ -23,8 +22,8 @@ namespace cmdg {
 
 // per-element record: xi11, xi22, xi33, J, sJ (6 faces), Delta
 constexpr int AFF_GEO = 11;
-// trace widths
-constexpr int TR_F2 = 4;  // second-order flux row d, states 1..4 (the mass entry is 0)
+// entries a face node
+constexpr int TR_F2 = 4;  // a second-order flux row: states 1..4 (the mass entry is 0)
 constexpr int TR_S = 2;   // Phi, p_ref
 
 struct AffArrays {
@@ -94,29 +93,25 @@ __device__ __forceinline__ double own_aux(const KParams &P, const double *__rest
 }
 
 // ------------------------------------------------------------------ gradient
-// Lifted-jump term Phi(n G*) - Phi(n G-) of face node fn of face f of element e
+// Lifted central jumps n (G* - G-) of face node fn of face f of element e
 // (DGModel_kernels.jl:1471-1647, CentralNumericalFluxGradient NumericalFluxes.jl:67-123,
-// walls: G* = n G(q_wall), bc_momentum.jl:24-43).  G- and theta_v- come from the
-// element's own gradient arguments in LDS, q+ from the neighbour's volume state.
+// walls: G* = n G(q_wall), bc_momentum.jl:24-43).  G- and theta_v- come from the element's
+// own gradient arguments in LDS, q+ from the neighbour's volume state.  A normal along axis d
+// fills row d of the gradient only, so four values carry the whole jump of the gradient
+// flux: u_c and h_tot here, and with a gravitational potential the fifth, N^2's
+// (row d of grad theta_v . grad Phi / theta_v); jump_gradient_flux spreads them.
 template <int Nq, bool SMAG, bool BUOY>
 __device__ __forceinline__ void face_gradient_aff(const KParams &P, const AffArrays &A, int64_t e, int f, int fn,
                                                   int32_t ne, const double *__restrict__ Q,
-                                                  const double (*sG)[Nq * Nq * Nq], double *dgf) {
-    constexpr int Np = Nq * Nq * Nq, Nfp = Nq * Nq, NG = SMAG ? 5 : 4, NGF = SMAG ? 10 : 9;
+                                                  const double (*sG)[Nq * Nq * Nq], double jump[5]) {
+    constexpr int Np = Nq * Nq * Nq, Nfp = Nq * Nq;
+    constexpr bool buoy = SMAG && BUOY;
     const int d = f >> 1, vn = face_node<Nq>(f, fn);
     const double nd = (f & 1) ? 1.0 : -1.0;
-    double G[5];
-#pragma unroll
-    for (int s = 0; s < 5; ++s) G[s] = s < NG ? sG[s][vn] : 0.0;
-    const double thv = SMAG ? G[4] : 0.0;
-    double gPhi[3] = {0.0, 0.0, 0.0};
     const int64_t ce = static_class(A, e);
-    if (P.a_gPhi >= 0) {
-        const double *ab = A.sa + (int64_t)Np * P.naux * ce + vn;
+    double G[5], Gp[5], Gs[5];
 #pragma unroll
-        for (int c = 0; c < 3; ++c) gPhi[c] = ab[(int64_t)Np * (P.a_gPhi + c)];
-    }
-    double Gp[5], Gs[5], nG[5];
+    for (int s = 0; s < 5; ++s) G[s] = (s < 4 || buoy) ? sG[s][vn] : 0.0;
     if (ne >= 0) {
         const int fo = f ^ 1;
         // the neighbour's state at the shared node, from its volume (the gradient pass
@@ -127,7 +122,7 @@ __device__ __forceinline__ void face_gradient_aff(const KParams &P, const AffArr
         for (int s = 0; s < 5; ++s) qp[s] = Q[qb + Np * s];
         const double Php = A.aux_cont ? own_aux<Nq>(P, A.sa, ce, vn, P.a_Phi, -0.0) : A.str[tri<Nfp>(ne, fo, 0, TR_S, fn)];
         Thermo tp = thermo(P, qp, Php);
-        grad_arg<SMAG>(P, qp, tp, SMAG ? (BUOY ? theta_v(P, tp) : 1.0) : 0.0, Gp);
+        grad_arg<buoy>(P, qp, tp, buoy ? theta_v(P, tp) : 0.0, Gp);
 #pragma unroll
         for (int s = 0; s < 5; ++s) Gs[s] = nd * (Gp[s] + G[s]) * 0.5;
     } else {
@@ -138,32 +133,67 @@ __device__ __forceinline__ void face_gradient_aff(const KParams &P, const AffArr
         const double nv[3] = {d == 0 ? nd : 0.0, d == 1 ? nd : 0.0, d == 2 ? nd : 0.0};
         wall_state(q, nv, 1.0, qb);
         Thermo tb = thermo(P, qb, Phi);
-        grad_arg<SMAG>(P, qb, tb, SMAG ? (BUOY ? theta_v(P, tb) : 1.0) : 0.0, Gp);
+        grad_arg<buoy>(P, qb, tb, buoy ? theta_v(P, tb) : 0.0, Gp);
 #pragma unroll
         for (int s = 0; s < 5; ++s) Gs[s] = nd * Gp[s];
     }
 #pragma unroll
-    for (int s = 0; s < 5; ++s) nG[s] = nd * G[s];
-    double gfs[10], gfm[10];
-    grad_flux_row<SMAG>(d, Gs, gPhi, thv, gfs);
-    grad_flux_row<SMAG>(d, nG, gPhi, thv, gfm);
-#pragma unroll
-    for (int s = 0; s < NGF; ++s) dgf[s] = gfs[s] - gfm[s];
+    for (int s = 0; s < 4; ++s) jump[s] = Gs[s] - nd * G[s];
+    if (buoy) {
+        const double gPd = A.sa[(int64_t)Np * (P.naux * ce + P.a_gPhi + d) + vn];
+        jump[4] = (Gs[4] * gPd) / G[4] - ((nd * G[4]) * gPd) / G[4];
+    }
 }
 
+// Adds w times the gradient-flux jump of a face along axis d (compile-time after unrolling)
+// to gf: the transform of a gradient with row d alone.  Halving is exact, so these are the
+// bits of transforming both sides and subtracting.
+template <bool BUOY>
+__device__ __forceinline__ void jump_gradient_flux(int d, double w, const double J[5], double *gf) {
+    gf[d] += w * J[3];
+    if (d == 0) {
+        gf[3] += w * J[0];
+        gf[4] += w * (J[1] * 0.5);
+        gf[5] += w * (J[2] * 0.5);
+    } else if (d == 1) {
+        gf[4] += w * (J[0] * 0.5);
+        gf[6] += w * J[1];
+        gf[7] += w * (J[2] * 0.5);
+    } else {
+        gf[5] += w * (J[0] * 0.5);
+        gf[7] += w * (J[1] * 0.5);
+        gf[8] += w * J[2];
+    }
+    if (BUOY) gf[9] += w * J[4];
+}
+
+// Viscosity planes (Np, viscosity_planes, nelem) beside the FP64 gradient flux: nu_d of
+// Smagorinsky-Lilly, 3 under a gravitational potential (the buoyancy correction makes it
+// anisotropic), 1 without; none for a constant viscosity, which the tendency has at hand.
+constexpr int viscosity_planes(bool smag, bool buoy) { return smag ? (buoy ? 3 : 1) : 0; }
+
 // BUOY: as for k_gradient_mix, theta_v and its gradient are evaluated for N^2 only when
-// the context has a gravitational potential.
+// the context has a gravitational potential.  Without one N^2 is zero, and its plane of the
+// gradient flux (which no kernel reads) is written with the auxiliary refresh only, in the
+// last pass of a call.
+// Bound by memory: 40 B a node read, 80 written, and the neighbours' lines.  It writes no
+// face trace: the tendency forms the neighbour's second-order row from the gradient flux
+// and the viscosity planes (8 B a node), where a trace of rows took 38.4 B a node written
+// here and read there; and a face's jump is the four or five values that differ from zero,
+// 4.8-6 KB of LDS instead of 12.  48^3 Smagorinsky-Lilly: 697 -> 579 us a launch (the
+// tendency 1005 -> 1017), 25^3 with gravity 120 -> 106 (151 -> 151), 33^3 constant
+// viscosity 242 -> 199 (338 -> 366).  Register caps of 96 and 80 spill (15 and 37
+// registers) and cost 763 and 1173 us at 48^3.
 template <int Nq, bool SMAG, bool BUOY>
 __global__ void __launch_bounds__(threads_for<Nq>())
 k_gradient_aff(KParams P, AffArrays A, ElemSet ES, const double *__restrict__ Q, double *__restrict__ aux,
-               double *__restrict__ gfo, double *__restrict__ f2tr, int write_aux) {
+               double *__restrict__ gfo, double *__restrict__ nuo, int write_aux) {
     constexpr int Np = Nq * Nq * Nq, Nfp = Nq * Nq, NT = threads_for<Nq>();
-    constexpr int NG = SMAG ? 5 : 4, NGF = SMAG ? 10 : 9;
+    constexpr bool buoy = SMAG && BUOY;
+    constexpr int NG = buoy ? 5 : 4, NGF = SMAG ? 10 : 9, NNU = viscosity_planes(SMAG, BUOY);
     __shared__ double sD[Nq * Nq];
-    __shared__ double sG[5][Np];
-    // lifted-jump terms (6 Nfp x NGF)
-    __shared__ double sJbuf[6 * Nfp * NGF];
-    double(*sJ)[NGF] = reinterpret_cast<double(*)[NGF]>(sJbuf);
+    __shared__ double sG[NG][Np];
+    __shared__ double sJ[NG][6 * Nfp];  // lifted jumps of the face nodes
     const int64_t e = set_element(ES, blockIdx.x);
     if (e < 0) return;
     __shared__ int32_t nb[6];  // the element's face neighbours
@@ -173,47 +203,47 @@ k_gradient_aff(KParams P, AffArrays A, ElemSet ES, const double *__restrict__ Q,
     const bool act = n < Np;
     const int i = n % Nq, j = (n / Nq) % Nq, k = n / (Nq * Nq);
     const double *ge = A.geo + (int64_t)AFF_GEO * e;
-    double q[5], thv = 0.0, G[5];
+    double rho = 0.0, thv = 1.0;
     Aux a;
-    constexpr bool buoy = SMAG && BUOY;
     if (act) {
         const double *qb = Q + (int64_t)Np * 5 * e + n;
+        double q[5], G[5];
 #pragma unroll
         for (int s = 0; s < 5; ++s) q[s] = qb[Np * s];
+        rho = q[0];
         a = load_aux(P, A.sa, Np, n, static_class(A, e));
         Thermo t = thermo(P, q, a.Phi);
         // theta_v enters N^2 = grad theta_v . grad Phi / theta_v only, zero without a
         // gravitational potential (grad Phi = 0): then it is evaluated only for the aux
-        // refresh, and 1 stands in the gradient argument (the face terms divide by it)
-        thv = (buoy || (write_aux && P.a_theta_v >= 0)) ? theta_v(P, t) : 1.0;
+        // refresh
+        if (buoy || (write_aux && P.a_theta_v >= 0)) thv = theta_v(P, t);
         if (write_aux) {
             double *ab = aux + (int64_t)Np * P.naux * e + n;
             if (P.a_theta_v >= 0) ab[(int64_t)Np * P.a_theta_v] = thv;
             if (P.a_air_T >= 0) ab[(int64_t)Np * P.a_air_T] = t.temp;
         }
-        grad_arg<SMAG>(P, q, t, thv, G);
+        grad_arg<buoy>(P, q, t, thv, G);
 #pragma unroll
         for (int s = 0; s < NG; ++s) sG[s][n] = G[s];
     }
     __syncthreads();
     // lifted central jumps of all face nodes, spread over every lane
     for (int t = n; t < 6 * Nfp; t += NT) {
-        double dgf[NGF];
-        face_gradient_aff<Nq, SMAG, BUOY>(P, A, e, t / Nfp, t % Nfp, nb[t / Nfp], Q, sG, dgf);
+        double J[5];
+        face_gradient_aff<Nq, SMAG, BUOY>(P, A, e, t / Nfp, t % Nfp, nb[t / Nfp], Q, sG, J);
 #pragma unroll
-        for (int s = 0; s < NGF; ++s) sJ[t][s] = dgf[s];
+        for (int s = 0; s < NG; ++s) sJ[s][t] = J[s];
     }
     __syncthreads();
 
-    double gf[10];
     if (act) {
         // horizontal pass then vertical pass, transform applied to each and summed
         const double xi0 = ge[0], xi1 = ge[1], xi2 = ge[2];
-        double gH[3][5], gV[3][5];
+        double gf[10], gH[3][5], gV[3][5];
 #pragma unroll
         for (int s = 0; s < 5; ++s) {
             double g1 = 0.0, g2 = 0.0, g3 = -0.0;
-            if (s < NG && (s < 4 || buoy)) {
+            if (s < NG) {
 #pragma unroll
                 for (int m = 0; m < Nq; ++m) {
                     g1 += sD[i + Nq * m] * sG[s][m + Nq * (j + Nq * k)];
@@ -230,10 +260,10 @@ k_gradient_aff(KParams P, AffArrays A, ElemSet ES, const double *__restrict__ Q,
             gV[2][s] = xi2 * g3;
         }
         double tmp[10];
-        grad_flux<SMAG>(gH, a, thv, gf);
-        grad_flux<SMAG>(gV, a, thv, tmp);
+        grad_flux<buoy>(gH, a, thv, gf);
+        grad_flux<buoy>(gV, a, thv, tmp);
 #pragma unroll
-        for (int s = 0; s < NGF; ++s) gf[s] += tmp[s];
+        for (int s = 0; s < (buoy ? 10 : 9); ++s) gf[s] += tmp[s];
         // the lifted jumps of this node's faces, in face order: M^-1 Mf (...)
         const double MI = 1.0 / (ge[3] * A.W[n]);
 #pragma unroll
@@ -242,27 +272,21 @@ k_gradient_aff(KParams P, AffArrays A, ElemSet ES, const double *__restrict__ Q,
             const int f = node_face_dir<Nq>(i, j, k, d, fn);
             if (f < 0) continue;
             const double w = MI * (ge[4 + f] * A.Wf[fn]);
+            double J[5];
 #pragma unroll
-            for (int s = 0; s < NGF; ++s) gf[s] += w * sJ[f * Nfp + fn][s];
+            for (int s = 0; s < NG; ++s) J[s] = sJ[s][f * Nfp + fn];
+            jump_gradient_flux<buoy>(d, w, J, gf);
         }
         double *go = gfo + (int64_t)Np * NGF * e + n;
 #pragma unroll
-        for (int s = 0; s < NGF; ++s) go[Np * s] = gf[s];
-    }
-    // the second-order flux rows of the face nodes, written straight to the face-major
-    // trace: the 25 lanes of one face fill its 25 contiguous slots per row entry
-    if (act && (i == 0 || i == Nq - 1 || j == 0 || j == Nq - 1 || k == 0 || k == Nq - 1)) {
-        double nu[3];
-        viscosity<SMAG>(P, q[0], gf, a.gPhi, ge[10], nu);
+        for (int s = 0; s < (buoy ? 10 : 9); ++s) go[Np * s] = gf[s];
+        if (SMAG) {
+            if (!buoy && write_aux) go[Np * 9] = 0.0;  // N^2
+            double nu[3];
+            viscosity<SMAG, BUOY>(P, rho, gf, a.gPhi, ge[10], nu);
+            double *no = nuo + (int64_t)Np * NNU * e + n;
 #pragma unroll
-        for (int d = 0; d < 3; ++d) {
-            int fn;
-            const int f = node_face_dir<Nq>(i, j, k, d, fn);
-            if (f < 0) continue;
-            double F2[5];
-            flux2_row<SMAG>(P, q, gf, nu, d, F2);
-#pragma unroll
-            for (int v = 0; v < TR_F2; ++v) f2tr[tri<Nfp>(e, f, v, TR_F2, fn)] = F2[1 + v];
+            for (int s = 0; s < NNU; ++s) no[Np * s] = nu[s];
         }
     }
 }
@@ -271,11 +295,16 @@ k_gradient_aff(KParams P, AffArrays A, ElemSet ES, const double *__restrict__ Q,
 // Numerical flux (first + second order, Rusanov or central) at face node fn of face
 // f of element e, seen from e (normal +-e_d): NumericalFluxes.jl:219-340, 670-715,
 // walls bc_momentum.jl:24-49 / bc_energy.jl:10-17 (zero second-order flux).
-template <int Nq, bool DIFF, bool SMAG>
+// The neighbour's second-order row is formed here from its gradient flux and viscosity at
+// the shared node (the strain-rate row, d h_tot / d x_d, nu_d; WithDivergence the two other
+// diagonal entries): the operations, and so the bits, of the neighbour's own row.
+template <int Nq, bool DIFF, int NNU>
 __device__ __forceinline__ void face_flux_aff(const KParams &P, const AffArrays &A, int f, int fn, int32_t ne,
-                                              const double (*sQ)[Nq * Nq * Nq],
-                                              const double *__restrict__ Q, const double *__restrict__ f2tr,
+                                              const double (*sQ)[Nq * Nq * Nq], const double *__restrict__ Q,
+                                              const double *__restrict__ gfi, const double *__restrict__ nui,
                                               const double *f2own, double flux[5]) {
+    constexpr bool SMAG = NNU > 0;
+    constexpr int NGF = SMAG ? 10 : 9;
     constexpr int Np = Nq * Nq * Nq, Nfp = Nq * Nq;
     const int d = f >> 1, vn = face_node<Nq>(f, fn);
     const double nd = (f & 1) ? 1.0 : -1.0;
@@ -289,14 +318,23 @@ __device__ __forceinline__ void face_flux_aff(const KParams &P, const AffArrays 
     for (int s = 0; s < 5; ++s) q[s] = sQ[s][vn];
     const double Phi = sQ[5][vn], ref_p = sQ[6][vn];
     double Php = Phi, refpp = ref_p;
-    double f2p[TR_F2] = {};  // the neighbour's second-order row, loaded with its state
+    // the neighbour's strain-rate row, trace, viscosity and enthalpy gradient, loaded with
+    // its state
+    double S0 = 0.0, S1 = 0.0, S2 = 0.0, trS = 0.0, nud = 0.0, gd = 0.0;
     if (!wall) {
         const double *qb = Q + (int64_t)Np * 5 * ne + face_node<Nq>(fo, fn);
 #pragma unroll
         for (int s = 0; s < 5; ++s) qp[s] = qb[Np * s];
-        if (DIFF)
-#pragma unroll
-            for (int v = 0; v < TR_F2; ++v) f2p[v] = f2tr[tri<Nfp>(ne, fo, v, TR_F2, fn)];
+        if (DIFF) {
+            const int vp = face_node<Nq>(fo, fn);
+            const double *gn = gfi + (int64_t)Np * NGF * ne + vp;
+            S0 = gn[Np * pick3(d, 3, 4, 5)];
+            S1 = gn[Np * pick3(d, 4, 6, 7)];
+            S2 = gn[Np * pick3(d, 5, 7, 8)];
+            gd = gn[Np * d];
+            if (SMAG) nud = nui[(int64_t)Np * (NNU * (int64_t)ne + (NNU == 3 ? d : 0)) + vp];
+            else if (P.with_div) trS = (gn[Np * 3] + gn[Np * 6]) + gn[Np * 8];
+        }
         if (!A.aux_cont) {
             Php = A.str[tri<Nfp>(ne, fo, 0, TR_S, fn)];
             refpp = A.str[tri<Nfp>(ne, fo, 1, TR_S, fn)];
@@ -326,12 +364,15 @@ __device__ __forceinline__ void face_flux_aff(const KParams &P, const AffArrays 
     }
     if (DIFF && !wall) {
         Fm[0] = 0.0;
-        Fp[0] = 0.0;
 #pragma unroll
-        for (int v = 0; v < TR_F2; ++v) {
-            Fm[1 + v] = f2own[v];  // the same bits the gradient kernel put in the trace
-            Fp[1 + v] = f2p[v];
+        for (int v = 0; v < TR_F2; ++v) Fm[1 + v] = f2own[v];
+        if (!SMAG) {
+            const double g0[1] = {0.0}, gP[3] = {0.0, 0.0, 0.0};
+            double nu[3];
+            viscosity<false>(P, qp[0], g0, gP, 0.0, nu);
+            nud = nu[0];
         }
+        flux2_row_parts<SMAG>(P, qp, S0, S1, S2, trS, nud, gd, d, Fp);
 #pragma unroll
         for (int s = 0; s < 5; ++s) flux[s] += (Fm[s] + Fp[s]) * h;
     }
@@ -343,13 +384,15 @@ __device__ __forceinline__ void face_flux_aff(const KParams &P, const AffArrays 
 //   or beta = 0 when dQ holds zeros (the previous stage scaled it by rka = 0): it is then
 //   not read; dq_store = 0 leaves the scaled dQ unstored (this stage's rka is 0 and the
 //   next stage is launched with beta = 0).
-template <int Nq, bool DIFF, bool SMAG, int MODE>
+// NNU: viscosity planes of nui (Smagorinsky-Lilly; 0: a constant viscosity).
+template <int Nq, bool DIFF, int NNU, int MODE>
 __global__ void __launch_bounds__(threads_for<Nq>())
 k_tendency_aff(KParams P, AffArrays A, ElemSet ES, const double *__restrict__ Q,
-               const double *__restrict__ gfi, const double *__restrict__ f2tr, double *__restrict__ aux,
+               const double *__restrict__ gfi, const double *__restrict__ nui, double *__restrict__ aux,
                double *__restrict__ tend, double alpha, double beta, double *__restrict__ Qout, double rka,
                double bdt, int write_aux, int dq_store) {
     constexpr int Np = Nq * Nq * Nq, Nfp = Nq * Nq, NT = threads_for<Nq>();
+    constexpr bool SMAG = NNU > 0;
     constexpr int NGF = SMAG ? 10 : 9;
     __shared__ double sD[Nq * Nq];
     // M(xi_a F) by direction; once every lane has its volume divergence (in registers),
@@ -370,14 +413,13 @@ k_tendency_aff(KParams P, AffArrays A, ElemSet ES, const double *__restrict__ Q,
     const int i = n % Nq, j = (n / Nq) % Nq, k = n / (Nq * Nq);
     const double *ge = A.geo + (int64_t)AFF_GEO * e;
 
-    double q[5], gf[10], u[3], nu[3], p = 0.0, pm = 0.0, MI = 0.0;
+    double q[5], gf[9], u[3], nu[3], p = 0.0, pm = 0.0, MI = 0.0;
     Aux a;
     if (act) {
         const double *qb = Q + (int64_t)Np * 5 * e + n;
 #pragma unroll
         for (int s = 0; s < 5; ++s) q[s] = qb[Np * s];
         a = load_aux(P, A.sa, Np, n, static_class(A, e));
-        a.Delta = ge[10];
         Thermo t = thermo(P, q, a.Phi);
         if (write_aux) {
             double *ab = aux + (int64_t)Np * P.naux * e + n;
@@ -392,8 +434,14 @@ k_tendency_aff(KParams P, AffArrays A, ElemSet ES, const double *__restrict__ Q,
         if (DIFF) {
             const double *gb = gfi + (int64_t)Np * NGF * e + n;
 #pragma unroll
-            for (int s = 0; s < NGF; ++s) gf[s] = gb[Np * s];
-            viscosity<SMAG>(P, q[0], gf, a.gPhi, a.Delta, nu);
+            for (int s = 0; s < 9; ++s) gf[s] = gb[Np * s];
+            if (SMAG) {
+                const double *nb_ = nui + (int64_t)Np * NNU * e + n;
+#pragma unroll
+                for (int d = 0; d < 3; ++d) nu[d] = nb_[Np * (NNU == 3 ? d : 0)];
+            } else {
+                viscosity<false>(P, q[0], gf, a.gPhi, 0.0, nu);
+            }
         }
         const double M = ge[3] * A.W[n];
         MI = 1.0 / M;
@@ -463,8 +511,8 @@ k_tendency_aff(KParams P, AffArrays A, ElemSet ES, const double *__restrict__ Q,
     // numerical fluxes of all face nodes, spread over every lane
     for (int t = n; t < 6 * Nfp; t += NT) {
         double fl5[5];
-        face_flux_aff<Nq, DIFF, SMAG>(P, A, t / Nfp, t % Nfp, nb[t / Nfp], sQ, Q, f2tr, sF2o[DIFF ? t : 0],
-                                      fl5);
+        face_flux_aff<Nq, DIFF, NNU>(P, A, t / Nfp, t % Nfp, nb[t / Nfp], sQ, Q, gfi, nui, sF2o[DIFF ? t : 0],
+                                     fl5);
 #pragma unroll
         for (int s = 0; s < 5; ++s) sFl[t][s] = fl5[s];
     }

@@ -279,7 +279,9 @@ __device__ __forceinline__ void flux1_row(const double q[5], const double u[3], 
 }
 
 // Diagonal of the kinematic viscosity tensor (TurbulenceClosures.jl:378-404, 472-499).
-template <bool SMAG>
+// BUOY false: no gravitational potential, so k = 0 and the buoyancy factor drops out:
+// nu_d = (nu_0 - 0) + 0 f_b = nu_0 exactly, formed without N^2, Ri or f_b.
+template <bool SMAG, bool BUOY = true>
 __device__ __forceinline__ void viscosity(const KParams &P, double rho, const double *gf, const double gPhi[3],
                                           double Delta, double nu[3]) {
     if (SMAG) {
@@ -287,11 +289,15 @@ __device__ __forceinline__ void viscosity(const KParams &P, double rho, const do
         double norm2 = ((((S[0] * S[0] + 2.0 * (S[1] * S[1])) + 2.0 * (S[2] * S[2])) + S[3] * S[3]) +
                         2.0 * (S[4] * S[4])) + S[5] * S[5];
         double normS = sqrt(2.0 * norm2);
+        double CD = P.C_smag * Delta;
+        double nu0 = normS * (CD * CD) + 1e-5;
+        if (!BUOY) {
+            nu[0] = nu[1] = nu[2] = nu0;
+            return;
+        }
         double k[3] = {gPhi[0] / P.grav, gPhi[1] / P.grav, gPhi[2] / P.grav};
         double Ri = gf[9] / (normS * normS + ulp_above(normS));
         double fb2 = sqrt(fmin(fmax(1.0 - Ri * P.inv_Pr, 0.0), 1.0));
-        double CD = P.C_smag * Delta;
-        double nu0 = normS * (CD * CD) + 1e-5;
         double dotk = (nu0 * k[0] + nu0 * k[1]) + nu0 * k[2];
 #pragma unroll
         for (int d = 0; d < 3; ++d) {
@@ -304,19 +310,16 @@ __device__ __forceinline__ void viscosity(const KParams &P, double rho, const do
     }
 }
 
-// Row d of the second-order flux (tendencies_momentum.jl:37-42, tendencies_energy.jl:27-56):
+// Row d of the second-order flux (tendencies_momentum.jl:37-42, tendencies_energy.jl:27-56)
+// from row d of the strain rate (S0, S1, S2), its trace (read WithDivergence only), nu_d
+// and d h_tot / d x_d:
 // tau[d][c] = -2 nu_d S[d][c] (+ 2 nu / 3 tr S on the diagonal WithDivergence).
 template <bool SMAG>
-__device__ __forceinline__ void flux2_row(const KParams &P, const double q[5], const double *gf, const double nu[3],
-                                          int d, double F[5]) {
-    const double *S = gf + 3;
-    const double S0 = pick3(d, S[0], S[1], S[2]);
-    const double S1 = pick3(d, S[1], S[3], S[4]);
-    const double S2 = pick3(d, S[2], S[4], S[5]);
-    const double nud = pick3(d, nu[0], nu[1], nu[2]);
+__device__ __forceinline__ void flux2_row_parts(const KParams &P, const double q[5], double S0, double S1, double S2,
+                                                double trS, double nud, double gd, int d, double F[5]) {
     double t0 = (-2.0 * nud) * S0, t1 = (-2.0 * nud) * S1, t2 = (-2.0 * nud) * S2;
     if (!SMAG && P.with_div) {
-        const double dv = ((2.0 * nud) / 3.0) * ((S[0] + S[3]) + S[5]);
+        const double dv = ((2.0 * nud) / 3.0) * trS;
         if (d == 0) t0 = t0 + dv;
         if (d == 1) t1 = t1 + dv;
         if (d == 2) t2 = t2 + dv;
@@ -326,23 +329,16 @@ __device__ __forceinline__ void flux2_row(const KParams &P, const double q[5], c
     F[2] = t1 * q[0];
     F[3] = t2 * q[0];
     const double vf = (t0 * q[1] + t1 * q[2]) + t2 * q[3];
-    const double gd = pick3(d, gf[0], gf[1], gf[2]);
     F[4] = vf + ((-(nud * P.inv_Pr)) * gd) * q[0];
 }
 
-// Gradient-flux transform of n (x) X with n = +-e_d (only row d of the 3 x 5 argument is non-zero).
+// the same from the node's gradient flux and viscosity
 template <bool SMAG>
-__device__ __forceinline__ void grad_flux_row(int d, const double X[5], const double gPhi[3], double thv, double *gf) {
-    double g[3][5];
-#pragma unroll
-    for (int r = 0; r < 3; ++r)
-#pragma unroll
-        for (int s = 0; s < 5; ++s) g[r][s] = (r == d) ? X[s] : 0.0;
-    Aux a;
-    a.gPhi[0] = gPhi[0];
-    a.gPhi[1] = gPhi[1];
-    a.gPhi[2] = gPhi[2];
-    grad_flux<SMAG>(g, a, thv, gf);
+__device__ __forceinline__ void flux2_row(const KParams &P, const double q[5], const double *gf, const double nu[3],
+                                          int d, double F[5]) {
+    const double *S = gf + 3;
+    flux2_row_parts<SMAG>(P, q, pick3(d, S[0], S[1], S[2]), pick3(d, S[1], S[3], S[4]), pick3(d, S[2], S[4], S[5]),
+                          (S[0] + S[3]) + S[5], pick3(d, nu[0], nu[1], nu[2]), pick3(d, gf[0], gf[1], gf[2]), d, F);
 }
 
 }  // namespace cmdg
