@@ -749,11 +749,12 @@ int create_impl(const cmdg_desc *d, const cmdg_brick *brick, void *stream, cmdg_
             // tiled traversal.  CMDG_ELEMENT_TILE=T sets cubic tiles of edge T (0 keeps
             // the storage order) and "TX,TY,TZ" tile extents along x, y, z (0: the whole
             // axis); CMDG_TILED_PASSES = tendency, gradient, both or none chooses the passes
-            // that walk the tiles.  Default: the tendency pass walks 8^3 tiles.  A mixed
-            // context whose face neighbours would, in storage order, leave one XCD's L2
+            // that walk the tiles.  Default: an FP64 context's tendency pass walks 8 x 8
+            // columns of elements spanning the whole y axis, a mixed context's 8^3 tiles.  A
+            // mixed context whose face neighbours would, in storage order, leave one XCD's L2
             // before the gradient pass gathers their state (the 90th percentile of the
             // storage distance between face neighbours, in state bytes, above 4 MiB) walks
-            // 12 x 12 columns of elements spanning the whole y axis, in both passes.
+            // 12 x 12 columns spanning y in both passes.
             // Measured on one box, chosen form (mixed + learned closure):
             //   96^3 (distance 9216 elements, 46 MB): tendency pass in 8^3 tiles 55.0 GDOF/s;
             //     both passes in 8^3 tiles 55.7-56.0 (edge 6 / 12 / 16: 55.3 / 56.2 / 55.8);
@@ -761,9 +762,10 @@ int create_impl(const cmdg_desc *d, const cmdg_brick *brick, void *stream, cmdg_
             //     mixed + Smagorinsky-Lilly 59.6 / 60.3 / 60.3;
             //   25^3 (625 elements, 3.1 MB): tendency pass in 8^3 tiles 50.0-50.3; both
             //     passes 49.3; 12 x 12 columns 49.2 (tendency pass), 48.6 (both).
-            // FP64 at 96^3: 40.1-40.4 with the tendency pass in 8^3 tiles (12 x 12 columns
-            // 40.2), 37.6-38.6 with both: its gradient pass, which writes the second-order
-            // face trace, loses in tiles more than its gathers gain.
+            // FP64 tendency, us a launch in 8^3 tiles / 6 x 6 / 8 x 8 columns: 64^3 2299 /
+            // 2338 / 2258, 48^3 977 / 943 / 965, 32^3 297 / 298 / 286, 33^3 347 / 343 / 341,
+            // 37 x 52 x 43 743 / 749 / 740, 25^3 131 / 130 / 130.  FP64 gradient: storage
+            // order 579 at 48^3, any tile 618-640.
             bool far = false;
             if (d->precision == CMDG_MIXED) {
                 std::vector<int64_t> gap;
@@ -778,7 +780,7 @@ int create_impl(const cmdg_desc *d, const cmdg_brick *brick, void *stream, cmdg_
                 }
             }
             const char *tile_env = std::getenv("CMDG_ELEMENT_TILE");
-            int T[3] = {8, 8, 8};
+            int T[3] = {8, d->precision == CMDG_MIXED ? 8 : 0, 8};
             if (far) T[0] = 12, T[1] = 0, T[2] = 12;
             if (tile_env && std::strchr(tile_env, ',')) {
                 if (std::sscanf(tile_env, "%d,%d,%d", &T[0], &T[1], &T[2]) != 3) T[0] = T[1] = T[2] = -1;

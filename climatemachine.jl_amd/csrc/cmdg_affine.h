@@ -299,8 +299,8 @@ k_gradient_aff(KParams P, AffArrays A, ElemSet ES, const double *__restrict__ Q,
 // the shared node (the strain-rate row, d h_tot / d x_d, nu_d; WithDivergence the two other
 // diagonal entries): the operations, and so the bits, of the neighbour's own row.
 template <int Nq, bool DIFF, int NNU>
-__device__ __forceinline__ void face_flux_aff(const KParams &P, const AffArrays &A, int f, int fn, int32_t ne,
-                                              const double (*sQ)[Nq * Nq * Nq], const double *__restrict__ Q,
+__device__ __forceinline__ void face_flux_aff(const KParams &P, const AffArrays &A, int64_t ce, int f, int fn,
+                                              int32_t ne, const double (*sQ)[Nq * Nq * Nq], const double *__restrict__ Q,
                                               const double *__restrict__ gfi, const double *__restrict__ nui,
                                               const double *f2own, double flux[5]) {
     constexpr bool SMAG = NNU > 0;
@@ -311,12 +311,13 @@ __device__ __forceinline__ void face_flux_aff(const KParams &P, const AffArrays 
     const double h = nd * 0.5;
     const bool wall = ne < 0;
     const int fo = f ^ 1;
-    // the own side at the face's volume node, staged in LDS (state rows 0-4, Phi 5,
-    // p_ref 6); the neighbour's state from its volume
+    // the own state at the face's volume node, staged in LDS; the neighbour's from its
+    // volume
     double q[5], qp[5];
 #pragma unroll
     for (int s = 0; s < 5; ++s) q[s] = sQ[s][vn];
-    const double Phi = sQ[5][vn], ref_p = sQ[6][vn];
+    const double Phi = own_aux<Nq>(P, A.sa, ce, vn, P.a_Phi, -0.0);
+    const double ref_p = own_aux<Nq>(P, A.sa, ce, vn, P.a_ref_p, 0.0);
     double Php = Phi, refpp = ref_p;
     // the neighbour's strain-rate row, trace, viscosity and enthalpy gradient, loaded with
     // its state
@@ -343,17 +344,32 @@ __device__ __forceinline__ void face_flux_aff(const KParams &P, const AffArrays 
         const double nv[3] = {d == 0 ? nd : 0.0, d == 1 ? nd : 0.0, d == 2 ? nd : 0.0};
         wall_state(q, nv, 2.0, qp);
     }
+    // the second-order part first: it leaves four values of the neighbour's six
+    double f2[TR_F2];
+    if (DIFF && !wall) {
+        double F2p[5];
+        if (!SMAG) {
+            const double g0[1] = {0.0}, gP[3] = {0.0, 0.0, 0.0};
+            double nu[3];
+            viscosity<false>(P, qp[0], g0, gP, 0.0, nu);
+            nud = nu[0];
+        }
+        flux2_row_parts<SMAG>(P, qp, S0, S1, S2, trS, nud, gd, d, F2p);
+#pragma unroll
+        for (int v = 0; v < TR_F2; ++v) f2[v] = (f2own[v] + F2p[1 + v]) * h;
+    }
+    __builtin_amdgcn_sched_barrier(0);
     const Thermo tm = thermo(P, q, Phi);
     const Thermo tp = thermo(P, qp, Php);
-    const double u[3] = {q[1] / q[0], q[2] / q[0], q[3] / q[0]};
-    const double up[3] = {qp[1] / qp[0], qp[2] / qp[0], qp[3] / qp[0]};
+    const double rim = 1.0 / q[0], rip = 1.0 / qp[0];
+    const double u[3] = {div_by(q[1], q[0], rim), div_by(q[2], q[0], rim), div_by(q[3], q[0], rim)};
+    const double up[3] = {div_by(qp[1], qp[0], rip), div_by(qp[2], qp[0], rip), div_by(qp[3], qp[0], rip)};
     double Fm[5], Fp[5];
     flux1_row(q, u, tm.p, P.ref_sub ? (tm.p - ref_p) : tm.p, d, Fm);
     flux1_row(qp, up, tp.p, P.ref_sub ? (tp.p - refpp) : tp.p, d, Fp);
 #pragma unroll
     for (int s = 0; s < 5; ++s) flux[s] = (Fm[s] + Fp[s]) * h;
     if (P.rusanov) {
-        const double rim = 1.0 / q[0], rip = 1.0 / qp[0];
         const double qmd = pick3(d, q[1], q[2], q[3]);
         const double qpd = pick3(d, qp[1], qp[2], qp[3]);
         const double wm = fabs(nd * (rim * qmd)) + sqrt(P.gammaR * tm.temp);
@@ -362,20 +378,9 @@ __device__ __forceinline__ void face_flux_aff(const KParams &P, const AffArrays 
 #pragma unroll
         for (int s = 0; s < 5; ++s) flux[s] += (mw * (q[s] - qp[s])) * 0.5;
     }
-    if (DIFF && !wall) {
-        Fm[0] = 0.0;
+    if (DIFF && !wall)
 #pragma unroll
-        for (int v = 0; v < TR_F2; ++v) Fm[1 + v] = f2own[v];
-        if (!SMAG) {
-            const double g0[1] = {0.0}, gP[3] = {0.0, 0.0, 0.0};
-            double nu[3];
-            viscosity<false>(P, qp[0], g0, gP, 0.0, nu);
-            nud = nu[0];
-        }
-        flux2_row_parts<SMAG>(P, qp, S0, S1, S2, trS, nud, gd, d, Fp);
-#pragma unroll
-        for (int s = 0; s < 5; ++s) flux[s] += (Fm[s] + Fp[s]) * h;
-    }
+        for (int v = 0; v < TR_F2; ++v) flux[1 + v] += f2[v];
 }
 
 // MODE 0: tend = alpha*RHS + beta*tend.   MODE 1: LSRK stage (tend is dQ):
@@ -385,8 +390,20 @@ __device__ __forceinline__ void face_flux_aff(const KParams &P, const AffArrays 
 //   not read; dq_store = 0 leaves the scaled dQ unstored (this stage's rka is 0 and the
 //   next stage is launched with beta = 0).
 // NNU: viscosity planes of nui (Smagorinsky-Lilly; 0: a constant viscosity).
+// What bounds it: nothing alone.  At 48^3 (Smagorinsky-Lilly) the lines that miss L2 are 290 B
+// a node read and 79 written, 5.1 TB/s; VALU issues in 45 % of the cycles, LDS in 27 %; each
+// wave waits two thirds of its life, so waves are what helps.  The horizontal fluxes share
+// one LDS space with the vertical ones and the staged state that follow them, and a face
+// node's own row shares its slot with the flux (16.2 KB a block; three directions at once
+// took 20.0), which with the second-order part of a face taken first (94 registers, 110-122
+// before) lets 5 waves a SIMD run instead of 4.  48^3: 1017 -> 965 us a launch, 33^3 constant
+// viscosity 366 -> 341, 25^3 with gravity 150.5 -> 147.5.  Fewer blocks a CU (LDS padding, 4
+// waves): 8 / 7 / 6 / 5 give 1010 / 1065 / 1150 / 1475 us; nine spilled registers 1332.  Face
+// tasks first, both sides read from memory instead of LDS, cut the missed lines to 213 B and
+// cost 1069 us: the added vector-memory instructions weigh more.
+// At Nq = 4 five waves spill.
 template <int Nq, bool DIFF, int NNU, int MODE>
-__global__ void __launch_bounds__(threads_for<Nq>())
+__global__ void __launch_bounds__(threads_for<Nq>()) __attribute__((amdgpu_waves_per_eu(Nq == 5 ? 5 : 4)))
 k_tendency_aff(KParams P, AffArrays A, ElemSet ES, const double *__restrict__ Q,
                const double *__restrict__ gfi, const double *__restrict__ nui, double *__restrict__ aux,
                double *__restrict__ tend, double alpha, double beta, double *__restrict__ Qout, double rka,
@@ -395,14 +412,13 @@ k_tendency_aff(KParams P, AffArrays A, ElemSet ES, const double *__restrict__ Q,
     constexpr bool SMAG = NNU > 0;
     constexpr int NGF = SMAG ? 10 : 9;
     __shared__ double sD[Nq * Nq];
-    // M(xi_a F) by direction; once every lane has its volume divergence (in registers),
-    // the same space holds the face fluxes (6 Nfp x 5) and the element's state, Phi and
-    // p_ref for the face tasks (7 x Np), so that the block needs no more LDS
-    __shared__ double sF[3][5][Np];
-    static_assert(6 * Nfp * 5 + 7 * Np <= 3 * 5 * Np, "face fluxes and staged state fit in sF");
-    double(*sFl)[5] = reinterpret_cast<double(*)[5]>(&sF[0][0][0]);
-    double(*sQ)[Np] = reinterpret_cast<double(*)[Np]>(&sF[0][0][0] + 6 * Nfp * 5);
-    __shared__ double sF2o[DIFF ? 6 * Nfp : 1][TR_F2];  // this element's rows at its face nodes
+    // M(xi_a F) of the two horizontal directions; then, once every lane has its horizontal
+    // divergence, of the vertical one (in [0]) and the element's state for the face tasks
+    // (in [1])
+    __shared__ double sF[2][5][Np];
+    double(*sQ)[Np] = sF[1];
+    // per face node: this element's second-order row, then the face flux in its place
+    __shared__ double sFl[6 * Nfp][5];
     const int64_t e = set_element(ES, blockIdx.x);
     if (e < 0) return;
     __shared__ int32_t nb[6];  // the element's face neighbours
@@ -413,24 +429,24 @@ k_tendency_aff(KParams P, AffArrays A, ElemSet ES, const double *__restrict__ Q,
     const int i = n % Nq, j = (n / Nq) % Nq, k = n / (Nq * Nq);
     const double *ge = A.geo + (int64_t)AFF_GEO * e;
 
-    double q[5], gf[9], u[3], nu[3], p = 0.0, pm = 0.0, MI = 0.0;
-    Aux a;
+    const int64_t ce = static_class(A, e);
+    double q[5], gf[9], u[3], nu[3], Fv[5], MI = 0.0;
     if (act) {
         const double *qb = Q + (int64_t)Np * 5 * e + n;
 #pragma unroll
         for (int s = 0; s < 5; ++s) q[s] = qb[Np * s];
-        a = load_aux(P, A.sa, Np, n, static_class(A, e));
-        Thermo t = thermo(P, q, a.Phi);
+        const Thermo t = thermo(P, q, own_aux<Nq>(P, A.sa, ce, n, P.a_Phi, -0.0));
         if (write_aux) {
             double *ab = aux + (int64_t)Np * P.naux * e + n;
             if (P.a_theta_v >= 0) ab[(int64_t)Np * P.a_theta_v] = theta_v(P, t);
             if (P.a_air_T >= 0) ab[(int64_t)Np * P.a_air_T] = t.temp;
         }
-        p = t.p;
-        pm = P.ref_sub ? (p - a.ref_p) : p;
-        u[0] = q[1] / q[0];
-        u[1] = q[2] / q[0];
-        u[2] = q[3] / q[0];
+        const double p = t.p;
+        const double pm = P.ref_sub ? (p - own_aux<Nq>(P, A.sa, ce, n, P.a_ref_p, 0.0)) : p;
+        const double rinv = 1.0 / q[0];
+        u[0] = div_by(q[1], q[0], rinv);
+        u[1] = div_by(q[2], q[0], rinv);
+        u[2] = div_by(q[3], q[0], rinv);
         if (DIFF) {
             const double *gb = gfi + (int64_t)Np * NGF * e + n;
 #pragma unroll
@@ -440,7 +456,8 @@ k_tendency_aff(KParams P, AffArrays A, ElemSet ES, const double *__restrict__ Q,
 #pragma unroll
                 for (int d = 0; d < 3; ++d) nu[d] = nb_[Np * (NNU == 3 ? d : 0)];
             } else {
-                viscosity<false>(P, q[0], gf, a.gPhi, 0.0, nu);
+                const double gP[3] = {0.0, 0.0, 0.0};
+                viscosity<false>(P, q[0], gf, gP, 0.0, nu);
             }
         }
         const double M = ge[3] * A.W[n];
@@ -455,26 +472,23 @@ k_tendency_aff(KParams P, AffArrays A, ElemSet ES, const double *__restrict__ Q,
                 const int f = node_face_dir<Nq>(i, j, k, ax, fn);
                 if (f >= 0)
 #pragma unroll
-                    for (int v = 0; v < TR_F2; ++v) sF2o[f * Nfp + fn][v] = F2[1 + v];
+                    for (int v = 0; v < TR_F2; ++v) sFl[f * Nfp + fn][v] = F2[1 + v];
 #pragma unroll
                 for (int s = 0; s < 5; ++s) F[s] += F2[s];
             }
             const double x = ge[ax];
 #pragma unroll
-            for (int s = 0; s < 5; ++s) sF[ax][s][n] = M * (x * F[s]);
+            for (int s = 0; s < 5; ++s) {
+                const double v = M * (x * F[s]);
+                if (ax < 2) sF[ax][s][n] = v;
+                else Fv[s] = v;
+            }
         }
     }
     __syncthreads();
-    // volume divergence and source of this node, into registers
+    // horizontal divergence of this node, into registers
     double T[5];
     if (act) {
-        double src[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-        if (P.gravity) {
-            // Gravity() source (tendencies_momentum.jl:60-72)
-            const double drho = P.ref_src ? (q[0] - a.ref_rho) : q[0];
-#pragma unroll
-            for (int d = 0; d < 3; ++d) src[1 + d] = (-drho) * a.gPhi[d];
-        }
         const double *tb = tend + (int64_t)Np * 5 * e + n;
 #pragma unroll
         for (int s = 0; s < 5; ++s) {
@@ -488,31 +502,49 @@ k_tendency_aff(KParams P, AffArrays A, ElemSet ES, const double *__restrict__ Q,
             // beta also bounds the scheduler: without it every LDS read of the five
             // variables is hoisted ahead of the arithmetic (224 VGPRs against 119,
             // occupancy 2 against 4 waves per SIMD).
-            const double out =
+            T[s] =
                 (beta != 0.0) ? alpha * th + beta * (MODE == 1 ? __builtin_nontemporal_load(tb + Np * s) : tb[Np * s])
                               : alpha * th;
+        }
+    }
+    __syncthreads();
+    if (act) {
+#pragma unroll
+        for (int s = 0; s < 5; ++s) {
+            sF[0][s][n] = Fv[s];
+            sQ[s][n] = q[s];
+        }
+    }
+    __syncthreads();
+    // vertical divergence and source
+    if (act) {
+        double src[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+        if (P.gravity) {
+            // Gravity() source (tendencies_momentum.jl:60-72), its static fields read again
+            // (a class's block stays in cache) rather than held across the barriers
+            const Aux a = load_aux(P, A.sa, Np, n, ce);
+            const double drho = P.ref_src ? (sQ[0][n] - a.ref_rho) : sQ[0][n];
+#pragma unroll
+            for (int d = 0; d < 3; ++d) src[1 + d] = (-drho) * a.gPhi[d];
+        }
+#pragma unroll
+        for (int s = 0; s < 5; ++s) {
             double tv = 0.0;
 #pragma unroll
             for (int m = 0; m < Nq; ++m) {
-                tv += MI * sD[m + Nq * k] * sF[2][s][i + Nq * (j + Nq * m)];
+                tv += MI * sD[m + Nq * k] * sF[0][s][i + Nq * (j + Nq * m)];
                 if (m == k) tv += src[s];
             }
-            T[s] = (MODE == 0 ? alpha * tv : tv) + out;
+            T[s] = (MODE == 0 ? alpha * tv : tv) + T[s];
         }
     }
-    __syncthreads();  // every read of sF is done: it now holds the staged state, then face fluxes
-    if (act) {
-#pragma unroll
-        for (int s = 0; s < 5; ++s) sQ[s][n] = q[s];
-        sQ[5][n] = a.Phi;
-        sQ[6][n] = a.ref_p;
-    }
-    __syncthreads();
     // numerical fluxes of all face nodes, spread over every lane
     for (int t = n; t < 6 * Nfp; t += NT) {
-        double fl5[5];
-        face_flux_aff<Nq, DIFF, NNU>(P, A, t / Nfp, t % Nfp, nb[t / Nfp], sQ, Q, gfi, nui, sF2o[DIFF ? t : 0],
-                                     fl5);
+        double own[TR_F2], fl5[5];
+        if (DIFF)
+#pragma unroll
+            for (int v = 0; v < TR_F2; ++v) own[v] = sFl[t][v];
+        face_flux_aff<Nq, DIFF, NNU>(P, A, ce, t / Nfp, t % Nfp, nb[t / Nfp], sQ, Q, gfi, nui, own, fl5);
 #pragma unroll
         for (int s = 0; s < 5; ++s) sFl[t][s] = fl5[s];
     }

@@ -36,6 +36,17 @@ struct KArrays {
     int64_t nelem;
 };
 
+// a / b given rb, the correctly rounded 1 / b: the quotient a rb corrected by its exact
+// remainder (the last step of a Newton division), with the hardware's fix-up of zero,
+// infinite and NaN operands.  The remainder is exact, so the result is a / b (1 + 2^-105)
+// rounded once: the IEEE quotient, short of a quotient that close to a rounding boundary.
+// Four FP64 instructions where the division takes eleven (its range scaling serves
+// denormal and huge operands); the kernels divide a node's momentum by one density.
+__device__ __forceinline__ double div_by(double a, double b, double rb) {
+    const double q = a * rb;
+    return __builtin_amdgcn_div_fixup(__builtin_fma(__builtin_fma(-b, q, a), rb, q), b, a);
+}
+
 // ------------------------------------------------------------------ physics
 // Thermodynamics.jl dry relations as reached from src/Atmos/Model/moisture.jl:32-47
 // and thermo_states.jl:67-77.
@@ -49,7 +60,7 @@ __device__ __forceinline__ Thermo thermo(const KParams &P, const double q[5], do
     double rek = rinv * ((q[1] * q[1] + q[2] * q[2]) + q[3] * q[3]) * 0.5;
     double rep = q[0] * Phi;
     t.e_int = rinv * (q[4] - rek - rep);
-    t.temp = P.T_0 + t.e_int / P.cv_d;
+    t.temp = P.T_0 + div_by(t.e_int, P.cv_d, P.inv_cv);
     t.p = (P.R_d * q[0]) * t.temp;
     return t;
 }
