@@ -279,6 +279,18 @@ int launch_copy(cmdg_ctx *c, double *dst, const double *src, int64_t n) {
     return check_hip(c, hipGetLastError(), "copy launch");
 }
 
+// the loss gradient's two launches; work holds train_rows(batch) rows
+int launch_loss_grad(const float *params, const float *shift, const float *scale, const float *samples, int64_t ld,
+                     const int64_t *idx, int64_t batch, double inv_norm, float *grad, float *work,
+                     hipStream_t stream) {
+    const int64_t nb = train_rows(batch);
+    hipLaunchKernelGGL(k_mlp_grad, dim3((unsigned)nb), dim3(TRAIN_NT), 0, stream, params, shift, scale, samples, ld,
+                       idx, batch, (float)inv_norm, work);
+    if (hipGetLastError() != hipSuccess) return CMDG_EHIP;
+    hipLaunchKernelGGL(k_grad_reduce, dim3((GRAD_W + REDUCE_C - 1) / REDUCE_C), dim3(256), 0, stream, work, nb, grad);
+    return hipGetLastError() == hipSuccess ? CMDG_OK : CMDG_EHIP;
+}
+
 // Exact scale c with c * base[i] == vals[i] for all i (NaN if none near vals[0] / base[0]).
 double exact_scale(const double *vals, int64_t vstride, const double *base, int count) {
     double c0 = vals[0] / base[0];
@@ -1077,13 +1089,8 @@ int cmdg_mlp_loss_grad(const float *params, const float *shift, const float *sca
                        int64_t work_floats, void *stream) {
     if (batch <= 0 || !params || !shift || !scale || !samples || !grad || !work) return CMDG_EINVAL;
     if (!idx && batch > ld) return CMDG_EINVAL;
-    const int64_t nb = (batch + TRAIN_TB - 1) / TRAIN_TB;
-    if (nb * GRAD_W > work_floats) return CMDG_EINVAL;
-    hipLaunchKernelGGL(k_mlp_grad, dim3((unsigned)nb), dim3(TRAIN_TB), 0, (hipStream_t)stream, params, shift, scale,
-                       samples, ld, idx, batch, (float)inv_norm, work);
-    if (hipGetLastError() != hipSuccess) return CMDG_EHIP;
-    hipLaunchKernelGGL(k_grad_reduce, dim3((GRAD_W + 255) / 256), dim3(256), 0, (hipStream_t)stream, work, nb, grad);
-    return hipGetLastError() == hipSuccess ? CMDG_OK : CMDG_EHIP;
+    if ((batch + TRAIN_TB - 1) / TRAIN_TB * GRAD_W > work_floats) return CMDG_EINVAL;
+    return launch_loss_grad(params, shift, scale, samples, ld, idx, batch, inv_norm, grad, work, (hipStream_t)stream);
 }
 
 }  // extern "C"
@@ -1136,12 +1143,7 @@ int cmdg_mlp_loss_grad_static(const float *params, const float *shift, const flo
     float *work = nullptr;
     const int rc = static_scratch((hipStream_t)stream, &work);
     if (rc) return rc;
-    const int64_t nb = (batch + TRAIN_TB - 1) / TRAIN_TB;
-    hipLaunchKernelGGL(k_mlp_grad, dim3((unsigned)nb), dim3(TRAIN_TB), 0, (hipStream_t)stream, params, shift, scale,
-                       samples, ld, idx, batch, (float)inv_norm, work);
-    if (hipGetLastError() != hipSuccess) return CMDG_EHIP;
-    hipLaunchKernelGGL(k_grad_reduce, dim3((GRAD_W + 255) / 256), dim3(256), 0, (hipStream_t)stream, work, nb, grad);
-    return hipGetLastError() == hipSuccess ? CMDG_OK : CMDG_EHIP;
+    return launch_loss_grad(params, shift, scale, samples, ld, idx, batch, inv_norm, grad, work, (hipStream_t)stream);
 }
 
 int cmdg_mlp_adam(float *params, const float *grad, float *m, float *v, int64_t n, float lr, float beta1, float beta2,

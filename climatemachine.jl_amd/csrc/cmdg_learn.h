@@ -218,7 +218,15 @@ __global__ void __launch_bounds__(128) k_element_average_pqr(float *__restrict__
 // b2 at 1376, W3 [32] at 1408, b3 at 1440.
 constexpr int MP_W1 = 0, MP_B1 = 320, MP_W2 = 352, MP_B2 = 1376, MP_W3 = 1408, MP_B3 = 1440, MLP_NPARAM = 1441;
 constexpr int GRAD_W = MLP_NPARAM + 1;  // + loss
-constexpr int TRAIN_TB = 64;            // samples per workgroup
+// A row of partial gradients is one workgroup's.  The caller's workspace holds a row for
+// every TRAIN_TB samples; a large batch fills TRAIN_ROWS of them, one a CU, and its waves take several
+// tiles each.
+constexpr int TRAIN_TB = 64, TRAIN_ROWS = 256;
+constexpr int TRAIN_NT = 256, TRAIN_TILE = 16;  // threads a workgroup; samples a wave's tile
+inline int64_t train_rows(int64_t batch) {
+    const int64_t nb = (batch + TRAIN_TB - 1) / TRAIN_TB;
+    return nb < TRAIN_ROWS ? nb : TRAIN_ROWS;
+}
 
 __device__ __forceinline__ float silu_fwd(float a, float &dsilu) {
 #pragma clang fp contract(fast)
@@ -227,94 +235,248 @@ __device__ __forceinline__ float silu_fwd(float a, float &dsilu) {
     return a * s;
 }
 
-// Per workgroup of 64 samples: the loss sum and its gradient with respect to every
-// parameter, written to partial[blockIdx][GRAD_W].  Forward as the inference (FP32
-// here, with the same input normalisation and output clamp), loss
+// The loss sum and its gradient with respect to every parameter over a workgroup's samples,
+// written to partial[blockIdx][GRAD_W].  Forward as the inference (FP32 here, with the same
+// input normalisation and output clamp), loss
 // sum_s (c^2 P + 2 c Q + R) * inv_norm, c = clamp(y, MLP_CMIN, MLP_CMAX).
-__global__ void __launch_bounds__(TRAIN_TB)
+//
+// Every product is a contraction, so it runs on FP32 MFMA (16x16x4: lane l holds
+// A[l%16][l/16], B[l/16][l%16] and D[4(l/16)..+3][l%16]; FP32 products and sums).  A wave
+// takes tiles of 16 samples as columns, features as rows: lane (g = l/16, s = l%16) holds
+// features 16m + 4g + r of sample s.  The sum over the features of the next layer may take
+// them in any order, so chunk (m, r) of it takes the features 16m + 4g + r, g = 0..3, that
+// the lanes already hold in register (m, r); only the weights are laid out to match.  The
+// weight gradients contract over samples, for which each matrix is transposed once through
+// the wave's LDS.  b1 rides along as the weight of an eleventh input that is 1.
+// 65536 rows of a 2^21-sample table: 188 -> 23 us (one lane a sample with its activations in
+// 170 registers ran one wave a SIMD, its weight-gradient loops 64 serial LDS reads long).
+// What is left is the gather (13 words of a sample lie in 13 lines): rows in order take 15.
+// 256 rows of partials, one workgroup a CU, are faster than 512 or 1024 from 32768 samples on
+// (27 against 31 and 33 us for the two launches at 65536), and equal below.
+__global__ void __launch_bounds__(TRAIN_NT)
 k_mlp_grad(const float *__restrict__ params, const float *__restrict__ shift, const float *__restrict__ scale,
            const float *__restrict__ samples, int64_t ld, const int64_t *__restrict__ idx, int64_t batch,
            float inv_norm, float *__restrict__ partial) {
 #pragma clang fp contract(fast)
-    __shared__ float sW[MLP_NPARAM];
-    __shared__ float sX[MLP_IN][TRAIN_TB], sH1[MLP_H][TRAIN_TB], sH2[MLP_H][TRAIN_TB];
-    __shared__ float sD1[MLP_H][TRAIN_TB], sD2[MLP_H][TRAIN_TB], sDy[TRAIN_TB], sL[TRAIN_TB];
-    const int t = threadIdx.x;
-    for (int q = t; q < MLP_NPARAM; q += TRAIN_TB) sW[q] = params[q];
-    __syncthreads();
-    const int64_t s = (int64_t)blockIdx.x * TRAIN_TB + t;
-    const bool valid = s < batch;
-    const int64_t row = valid ? (idx ? idx[s] : s) : 0;
-    float x[MLP_IN], P = 0.0f, Qv = 0.0f, R = 0.0f;
-    for (int k = 0; k < MLP_IN; ++k) {
-        x[k] = valid ? (samples[ld * k + row] - shift[k]) * scale[k] : 0.0f;
-        sX[k][t] = x[k];
+    constexpr int NW = TRAIN_NT / 64, LD = TRAIN_TILE + 1;     // a padded row of 16 samples
+    constexpr int R_D2 = 0, R_H1 = 32, R_D1 = 64, R_X = 96, ROWS = 112;
+    static_assert(ROWS * LD >= GRAD_W, "a wave's slab holds its gradient row at the end");
+    __shared__ float slab[NW][ROWS * LD];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, s = lane & 15, g = lane >> 4;
+    float *W = slab[wave];
+
+    // weights as MFMA operands, biases and w3 in the features' layout
+    float A1[2][3], A2[2][2][4], A2t[2][2][4], B2[2][4], W3[2][4];
+#pragma unroll
+    for (int m = 0; m < 2; ++m) {
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            const int k = 4 * c + g, o = 16 * m + s;
+            A1[m][c] = k < MLP_IN ? params[MP_W1 + MLP_IN * o + k] : (k == MLP_IN ? params[MP_B1 + o] : 0.0f);
+        }
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                A2[m][q][r] = params[MP_W2 + MLP_H * (16 * m + s) + 16 * q + 4 * g + r];
+                A2t[m][q][r] = params[MP_W2 + MLP_H * (16 * q + 4 * g + r) + 16 * m + s];
+            }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            B2[m][r] = params[MP_B2 + 16 * m + 4 * g + r];
+            W3[m][r] = params[MP_W3 + 16 * m + 4 * g + r];
+        }
     }
-    if (valid) {
-        P = samples[ld * 10 + row];
-        Qv = samples[ld * 11 + row];
-        R = samples[ld * 12 + row];
+    const float b3 = params[MP_B3];
+    float sh[3], sc[3];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+        const int k = 4 * c + g;
+        sh[c] = k < MLP_IN ? shift[k] : 0.0f;
+        sc[c] = k < MLP_IN ? scale[k] : 0.0f;
     }
-    float a1d[MLP_H], h1[MLP_H];
-    for (int o = 0; o < MLP_H; ++o) {
-        float a = sW[MP_B1 + o];
-        for (int k = 0; k < MLP_IN; ++k) a += sW[MP_W1 + MLP_IN * o + k] * x[k];
-        h1[o] = silu_fwd(a, a1d[o]);
-        sH1[o][t] = h1[o];
+
+    mlp_f32x4 G2[2][2] = {}, G1[2] = {};  // dW2 and dW1 (with db1) of the wave's samples
+    float g3[2][4] = {}, gb2[2][4] = {}, gb3 = 0.0f, loss = 0.0f;
+
+    // the four words of a sample that this lane reads: inputs g, 4 + g, 8 + g and row 10 + g
+    const int64_t ntile = (batch + TRAIN_TILE - 1) / TRAIN_TILE, stride = (int64_t)gridDim.x * NW;
+    float raw[4];
+    bool valid;
+    auto fetch = [&](int64_t tile) {
+        const int64_t i = tile * TRAIN_TILE + s;
+        valid = tile < ntile && i < batch;
+        raw[0] = raw[1] = raw[2] = raw[3] = 0.0f;
+        if (valid) {
+            const float *p = samples + (idx ? idx[i] : i);
+            raw[0] = p[ld * g];
+            raw[1] = p[ld * (4 + g)];
+            if (g < 2) raw[2] = p[ld * (8 + g)];
+            if (g < 3) raw[3] = p[ld * (10 + g)];
+        }
+    };
+    int64_t tile = (int64_t)blockIdx.x * NW + wave;
+    fetch(tile);
+    for (; tile < ntile; tile += stride) {
+        const bool live = valid;
+        float x[3];
+#pragma unroll
+        for (int c = 0; c < 3; ++c) x[c] = live ? (raw[c] - sh[c]) * sc[c] : 0.0f;
+        if (g == 2) x[2] = 1.0f;  // input 10
+        const float pqr = raw[3];
+        const float P = __shfl(pqr, s), Qv = __shfl(pqr, 16 + s), R = __shfl(pqr, 32 + s);
+        fetch(tile + stride);
+
+        float h1[2][4], a1d[2][4], a2d[2][4], y = 0.0f;
+#pragma unroll
+        for (int m = 0; m < 2; ++m) {
+            mlp_f32x4 a = {};
+#pragma unroll
+            for (int c = 0; c < 3; ++c) a = __builtin_amdgcn_mfma_f32_16x16x4f32(A1[m][c], x[c], a, 0, 0, 0);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) h1[m][r] = silu_fwd(a[r], a1d[m][r]);
+        }
+        float h2[2][4];
+#pragma unroll
+        for (int m = 0; m < 2; ++m) {
+            mlp_f32x4 a = {B2[m][0], B2[m][1], B2[m][2], B2[m][3]};
+#pragma unroll
+            for (int q = 0; q < 2; ++q)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    a = __builtin_amdgcn_mfma_f32_16x16x4f32(A2[m][q][r], h1[q][r], a, 0, 0, 0);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                h2[m][r] = silu_fwd(a[r], a2d[m][r]);
+                y += W3[m][r] * h2[m][r];
+            }
+        }
+        y += __shfl_xor(y, 16);
+        y += __shfl_xor(y, 32);
+        y += b3;
+        float dy = 0.0f;
+        if (live) {
+            const bool clamped = y > MLP_CMAX || y < MLP_CMIN;
+            const float c = fminf(fmaxf(y, MLP_CMIN), MLP_CMAX);
+            loss += (c * c * P + 2.0f * c * Qv + R) * inv_norm;
+            dy = clamped ? 0.0f : (2.0f * c * P + 2.0f * Qv) * inv_norm;
+        }
+        gb3 += dy;
+        float d2[2][4];
+#pragma unroll
+        for (int m = 0; m < 2; ++m)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                d2[m][r] = dy * W3[m][r] * a2d[m][r];
+                g3[m][r] += dy * h2[m][r];
+                gb2[m][r] += d2[m][r];
+                const int f = 16 * m + 4 * g + r;
+                W[(R_D2 + f) * LD + s] = d2[m][r];
+                W[(R_H1 + f) * LD + s] = h1[m][r];
+            }
+#pragma unroll
+        for (int c = 0; c < 3; ++c) W[(R_X + 4 * c + g) * LD + s] = x[c];
+        W[(R_X + 12 + g) * LD + s] = 0.0f;
+#pragma unroll
+        for (int m = 0; m < 2; ++m) {
+            mlp_f32x4 a = {};
+#pragma unroll
+            for (int q = 0; q < 2; ++q)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    a = __builtin_amdgcn_mfma_f32_16x16x4f32(A2t[m][q][r], d2[q][r], a, 0, 0, 0);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) W[(R_D1 + 16 * m + 4 * g + r) * LD + s] = a[r] * a1d[m][r];
+        }
+        // the slab is the wave's own: LDS serves one wave's accesses in order
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            float u2[2], u1[2], v2[2];
+#pragma unroll
+            for (int m = 0; m < 2; ++m) {
+                u2[m] = W[(R_D2 + 16 * m + s) * LD + 4 * c + g];
+                u1[m] = W[(R_D1 + 16 * m + s) * LD + 4 * c + g];
+                v2[m] = W[(R_H1 + 16 * m + s) * LD + 4 * c + g];
+            }
+            const float v1 = W[(R_X + s) * LD + 4 * c + g];
+#pragma unroll
+            for (int m = 0; m < 2; ++m) {
+                G1[m] = __builtin_amdgcn_mfma_f32_16x16x4f32(u1[m], v1, G1[m], 0, 0, 0);
+#pragma unroll
+                for (int q = 0; q < 2; ++q)
+                    G2[m][q] = __builtin_amdgcn_mfma_f32_16x16x4f32(u2[m], v2[q], G2[m][q], 0, 0, 0);
+            }
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     }
-    float a2d[MLP_H], y = sW[MP_B3];
-    for (int o = 0; o < MLP_H; ++o) {
-        float a = sW[MP_B2 + o];
-        for (int k = 0; k < MLP_H; ++k) a += sW[MP_W2 + MLP_H * o + k] * h1[k];
-        const float h2 = silu_fwd(a, a2d[o]);
-        sH2[o][t] = h2;
-        y += sW[MP_W3 + o] * h2;
+
+    // the wave's gradient row into its slab, then the workgroup's sum in wave order
+#pragma unroll
+    for (int m = 0; m < 2; ++m)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int o = 16 * m + 4 * g + r;
+            if (s < MLP_IN) W[MP_W1 + MLP_IN * o + s] = G1[m][r];
+            if (s == MLP_IN) W[MP_B1 + o] = G1[m][r];
+#pragma unroll
+            for (int q = 0; q < 2; ++q) W[MP_W2 + MLP_H * o + 16 * q + s] = G2[m][q][r];
+            float v3 = g3[m][r], vb = gb2[m][r];
+#pragma unroll
+            for (int w = 1; w < 16; w <<= 1) {
+                v3 += __shfl_xor(v3, w);
+                vb += __shfl_xor(vb, w);
+            }
+            if (s == 0) {
+                W[MP_W3 + o] = v3;
+                W[MP_B2 + o] = vb;
+            }
+        }
+#pragma unroll
+    for (int w = 1; w < 16; w <<= 1) {
+        gb3 += __shfl_xor(gb3, w);
+        loss += __shfl_xor(loss, w);
     }
-    float dy = 0.0f, L = 0.0f;
-    if (valid) {
-        const bool clamped = y > MLP_CMAX || y < MLP_CMIN;
-        const float c = fminf(fmaxf(y, MLP_CMIN), MLP_CMAX);
-        L = (c * c * P + 2.0f * c * Qv + R) * inv_norm;
-        dy = clamped ? 0.0f : (2.0f * c * P + 2.0f * Qv) * inv_norm;
+    if (lane == 0) {
+        W[MP_B3] = gb3;
+        W[MLP_NPARAM] = loss;
     }
-    sDy[t] = dy;
-    sL[t] = L;
-    float dh1[MLP_H];
-    for (int k = 0; k < MLP_H; ++k) dh1[k] = 0.0f;
-    for (int o = 0; o < MLP_H; ++o) {
-        const float d2 = dy * sW[MP_W3 + o] * a2d[o];
-        sD2[o][t] = d2;
-        for (int k = 0; k < MLP_H; ++k) dh1[k] += sW[MP_W2 + MLP_H * o + k] * d2;
-    }
-    for (int k = 0; k < MLP_H; ++k) sD1[k][t] = dh1[k] * a1d[k];
     __syncthreads();
     float *pb = partial + (int64_t)blockIdx.x * GRAD_W;
-    for (int q = t; q < GRAD_W; q += TRAIN_TB) {
-        const float *u, *v = nullptr;
-        if (q < MP_B1) { u = sD1[q / MLP_IN]; v = sX[q % MLP_IN]; }
-        else if (q < MP_W2) u = sD1[q - MP_B1];
-        else if (q < MP_B2) { const int r = q - MP_W2; u = sD2[r / MLP_H]; v = sH1[r % MLP_H]; }
-        else if (q < MP_W3) u = sD2[q - MP_B2];
-        else if (q < MP_B3) { u = sDy; v = sH2[q - MP_W3]; }
-        else if (q == MP_B3) u = sDy;
-        else u = sL;
-        float acc = 0.0f;
-        if (v)
-            for (int r = 0; r < TRAIN_TB; ++r) acc += u[r] * v[r];
-        else
-            for (int r = 0; r < TRAIN_TB; ++r) acc += u[r];
+    for (int q = threadIdx.x; q < GRAD_W; q += TRAIN_NT) {
+        float acc = slab[0][q];
+#pragma unroll
+        for (int w = 1; w < NW; ++w) acc += slab[w][q];
         pb[q] = acc;
     }
 }
 
-// grad[q] = sum over workgroups of partial[b][q], in workgroup order (deterministic);
-// the last entry is the loss.
-__global__ void k_grad_reduce(const float *__restrict__ partial, int64_t nb, float *__restrict__ grad) {
-    const int q = blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= GRAD_W) return;
+// grad[q] = sum over the rows of partial[b][q] in FP64, in a fixed order (deterministic): 16
+// columns a workgroup, 16 lanes a column, each every 16th row, then those 16 in order.  The
+// last entry is the loss.  (One lane a column took 250 us over 1024 rows: six workgroups,
+// one load after the other.)
+constexpr int REDUCE_C = 16;
+__global__ void __launch_bounds__(256) k_grad_reduce(const float *__restrict__ partial, int64_t nb,
+                                                     float *__restrict__ grad) {
+    __shared__ double red[16][REDUCE_C + 1];
+    const int c = threadIdx.x % REDUCE_C, r = threadIdx.x / REDUCE_C;
+    const int q = blockIdx.x * REDUCE_C + c;
     double acc = 0.0;
-    for (int64_t b = 0; b < nb; ++b) acc += partial[b * GRAD_W + q];
-    grad[q] = (float)acc;
+    if (q < GRAD_W) {
+#pragma unroll 8
+        for (int64_t b = r; b < nb; b += 16) acc += (double)partial[b * GRAD_W + q];
+    }
+    red[r][c] = acc;
+    __syncthreads();
+    if (r == 0 && q < GRAD_W) {
+#pragma unroll
+        for (int k = 1; k < 16; ++k) acc += red[k][c];
+        grad[q] = (float)acc;
+    }
 }
 
 __global__ void k_adam(float *__restrict__ p, const float *__restrict__ g, float *__restrict__ m,
