@@ -109,7 +109,7 @@ struct cmdg_ctx {
     // diagnostics (Courant numbers, weighted sums): reduction scratch, allocated on first use
     int32_t aux_coord = -1;
     double2 *d_part = nullptr;
-    double *d_scalar = nullptr;
+    double *h_scalar = nullptr, *d_scalar = nullptr;  // pinned, and as the device sees it
     int64_t npart = 0;
     std::string err;
     // optional per-kernel event timing (cmdg_set_kernel_timing)
@@ -905,7 +905,7 @@ int cmdg_destroy(cmdg_ctx *c) {
     (void)hipFree(c->d_gphi32);
     (void)hipFree(c->d_mlp);
     (void)hipFree(c->d_part);
-    (void)hipFree(c->d_scalar);
+    (void)hipHostFree(c->h_scalar);
     delete c;
     return CMDG_OK;
 }
@@ -1194,9 +1194,9 @@ static int diag_scratch(cmdg_ctx *c, int64_t n) {
 static int diag_result(cmdg_ctx *c, double *out) {
     int rc = check_hip(c, hipGetLastError(), "diagnostic launch");
     if (rc) return rc;
-    rc = check_hip(c, hipMemcpyAsync(out, c->d_scalar, sizeof(double), hipMemcpyDeviceToHost, c->stream), "hipMemcpyAsync");
-    if (rc) return rc;
-    return check_hip(c, hipStreamSynchronize(c->stream), "hipStreamSynchronize");
+    rc = check_hip(c, hipStreamSynchronize(c->stream), "hipStreamSynchronize");
+    if (!rc) *out = *c->h_scalar;
+    return rc;
 }
 
 int cmdg_courant(cmdg_ctx *c, const double *Q, double dt, int32_t kind, int32_t direction, double *out) {
@@ -1227,7 +1227,7 @@ int cmdg_courant(cmdg_ctx *c, const double *Q, double dt, int32_t kind, int32_t 
     else CMDG_COURANT_NQ(4);
 #undef CMDG_COURANT_NQ
 #undef CMDG_COURANT
-    hipLaunchKernelGGL(k_max_reduce, dim3(1), dim3(256), 0, c->stream, part, c->nelem, c->d_scalar);
+    hipLaunchKernelGGL(k_max_reduce, dim3(1), dim3(256), 0, c->stream, part, nb, c->d_scalar);
     return diag_result(c, out);
 }
 
@@ -1237,13 +1237,17 @@ int cmdg_weightedsum(cmdg_ctx *c, const double *Q, int32_t state, double *out) {
     if (state < 0 || state > 4) return fail(c, CMDG_EINVAL, "state index out of range");
     const int64_t total = (int64_t)c->Np * c->nelem;
     int64_t nb = (total + 255) / 256;
-    if (nb > 1024) nb = 1024;
+    if (nb > DIAG_BLOCKS) nb = DIAG_BLOCKS;
     int rc = diag_scratch(c, nb);
     if (rc) return rc;
     // M per node: vgeo's mass on general meshes; J w_i w_j w_k on affine bricks, which
     // the create-time check found equal to vgeo's M bit for bit
-    hipLaunchKernelGGL(k_weightedsum, dim3((unsigned)nb), dim3(256), 0, c->stream, Q, c->d_vg, c->Np, NVG,
-                       c->affine ? c->d_geo : nullptr, c->d_W, state, c->nelem, c->d_part);
+#define CMDG_WSUM(NQ)                                                                                             \
+    hipLaunchKernelGGL((k_weightedsum<NQ>), dim3((unsigned)nb), dim3(256), 0, c->stream, Q, c->d_vg, NVG,       \
+                       c->affine ? c->d_geo : nullptr, c->d_W, state, c->nelem, c->d_part)
+    if (c->Nq == 5) CMDG_WSUM(5);
+    else CMDG_WSUM(4);
+#undef CMDG_WSUM
     hipLaunchKernelGGL(k_dd_reduce, dim3(1), dim3(256), 0, c->stream, c->d_part, (int)nb, c->d_scalar);
     return diag_result(c, out);
 }
@@ -1253,7 +1257,7 @@ int cmdg_not_finite_fields(cmdg_ctx *c, const double *Q, int32_t *mask) {
     if (!Q || !mask) return fail(c, CMDG_EINVAL, "null pointer");
     const int64_t total = (int64_t)c->Np * 5 * c->nelem;
     int64_t nb = (total + 255) / 256;
-    if (nb > 1024) nb = 1024;
+    if (nb > DIAG_BLOCKS) nb = DIAG_BLOCKS;
     int rc = diag_scratch(c, nb);
     if (rc) return rc;
     hipLaunchKernelGGL(k_not_finite, dim3((unsigned)nb), dim3(256), 0, c->stream, Q, c->Np, 5, total, c->d_part);
