@@ -173,10 +173,10 @@ int launch_gradient_impl(cmdg_ctx *c, const double *Q, double *Qcopy, int write_
     const bool buoy = c->P.a_gPhi >= 0;
 #define CMDG_GRAD_MIX(SMAG, LEARN, BUOY)                                                                       \
     hipLaunchKernelGGL((k_gradient_mix<Nq, SMAG, LEARN, BUOY>), grid, block, 0, c->stream, c->P, c->MP, c->AA, ES, \
-                       Q, c->d_aux, c->d_gf32, write_aux, c->d_mlp)
+                       Q, c->d_aux, c->d_gf32, Qcopy, write_aux, c->d_mlp)
 #define CMDG_GRAD_AFF(SMAG, BUOY)                                                                               \
     hipLaunchKernelGGL((k_gradient_aff<Nq, SMAG, BUOY>), grid, block, 0, c->stream, c->P, c->AA, ES, Q, c->d_aux, \
-                       c->d_gf, c->d_nu, write_aux)
+                       c->d_gf, c->d_nu, Qcopy, write_aux)
     if (c->mixed) {
         if (c->learned) {
             if (buoy) CMDG_GRAD_MIX(true, true, true);
@@ -949,15 +949,21 @@ int cmdg_lsrk54_steps(cmdg_ctx *c, double *Q, double *dQ, double t, double dt, i
     // state to another buffer: the stages alternate between the caller's Q (C) and the
     // context buffer S, and no caller code runs between the steps of one call.  Over
     // 5 nsteps stages the result lands in C when that count is even; when it is odd,
-    // S <- C first (on general meshes by the first gradient pass) and the first stage
-    // reads S.
+    // S <- C first and the first stage reads S.  A diffusive context's first gradient pass
+    // reads C and writes the copy as it goes: 40 B a node and no launch, where a copy moves 80.
+    // One step, us, copy kernel / fused: FP64 25^3 1100 / 1095, 33^3 2702 / 2675, 48^3 8125 /
+    // 8048; mixed 16^3 277 / 275, 25^3 851 / 854, 30^3 1484 / 1493, 33^3 2085 / 2057, 64^3
+    // 15139 / 14885.  The mixed passes lose to those stores where the two states fit the
+    // last-level cache but not the L2s, 64 to 160 MiB a state: there the copy kernel stays.
+    const int64_t bytes = (int64_t)c->Np * 5 * c->nelem * (int64_t)sizeof(double), MiB = 1 << 20;
+    const bool fused_copy = c->diffusive && !(c->mixed && bytes > 64 * MiB && bytes <= 160 * MiB);
     double *C = Q, *S = c->d_Qs;
     double *src = C, *dst = S;
     const bool odd = (nsteps % 2) != 0;
     if (odd) {
         src = S;
         dst = C;
-        if ((c->affine || !c->diffusive) && (rc = launch_copy(c, S, C, (int64_t)c->Np * 5 * c->nelem))) return rc;
+        if (!fused_copy && (rc = launch_copy(c, S, C, (int64_t)c->Np * 5 * c->nelem))) return rc;
     }
     for (int64_t step = 0; step < nsteps; ++step)
         for (int s = 0; s < 5; ++s) {
@@ -974,7 +980,7 @@ int cmdg_lsrk54_steps(cmdg_ctx *c, double *Q, double *dQ, double t, double dt, i
             const double dq_read = (s == 0 && step > 0) ? 0.0 : 1.0;
             const int dq_store = !(s == 4 && step < nsteps - 1);
             if (c->diffusive) {
-                const bool first = odd && step == 0 && s == 0 && !c->affine;
+                const bool first = odd && fused_copy && step == 0 && s == 0;
                 if ((rc = launch_gradient(c, first ? C : src, first ? S : nullptr, wa))) return rc;
             }
             if ((rc = launch_tendency(c, src, dQ, 1.0, dq_read, 1, dst, a, bdt, c->diffusive ? 0 : wa, dq_store)))

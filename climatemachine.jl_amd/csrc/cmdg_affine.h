@@ -187,7 +187,7 @@ constexpr int viscosity_planes(bool smag, bool buoy) { return smag ? (buoy ? 3 :
 template <int Nq, bool SMAG, bool BUOY>
 __global__ void __launch_bounds__(threads_for<Nq>())
 k_gradient_aff(KParams P, AffArrays A, ElemSet ES, const double *__restrict__ Q, double *__restrict__ aux,
-               double *__restrict__ gfo, double *__restrict__ nuo, int write_aux) {
+               double *__restrict__ gfo, double *__restrict__ nuo, double *__restrict__ Qcopy, int write_aux) {
     constexpr int Np = Nq * Nq * Nq, Nfp = Nq * Nq, NT = threads_for<Nq>();
     constexpr bool buoy = SMAG && BUOY;
     constexpr int NG = buoy ? 5 : 4, NGF = SMAG ? 10 : 9, NNU = viscosity_planes(SMAG, BUOY);
@@ -210,6 +210,9 @@ k_gradient_aff(KParams P, AffArrays A, ElemSet ES, const double *__restrict__ Q,
         double q[5], G[5];
 #pragma unroll
         for (int s = 0; s < 5; ++s) q[s] = qb[Np * s];
+        if (Qcopy)  // the step's working copy of the state: written once, next read a pass later
+#pragma unroll
+            for (int s = 0; s < 5; ++s) __builtin_nontemporal_store(q[s], Qcopy + (int64_t)Np * (s + 5 * e) + n);
         rho = q[0];
         a = load_aux(P, A.sa, Np, n, static_class(A, e));
         Thermo t = thermo(P, q, a.Phi);

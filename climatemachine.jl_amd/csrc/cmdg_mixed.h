@@ -228,7 +228,8 @@ __device__ __forceinline__ void grad_arg_f(const KParams &P, const MixParams &M,
 template <int Nq, bool SMAG, bool LEARN, bool BUOY>
 __global__ void __launch_bounds__(threads_for<Nq>()) __attribute__((amdgpu_waves_per_eu(Nq == 5 ? 7 : 5)))
 k_gradient_mix(KParams P, MixParams MP, AffArrays A, ElemSet ES, const double *__restrict__ Q,
-               double *__restrict__ aux, float *__restrict__ gfo, int write_aux, const MlpDev *__restrict__ mlp) {
+               double *__restrict__ aux, float *__restrict__ gfo, double *__restrict__ Qcopy, int write_aux,
+               const MlpDev *__restrict__ mlp) {
 #pragma clang fp contract(fast)
     static_assert(!LEARN || SMAG, "the learned closure keeps the Smagorinsky-Lilly structure");
     constexpr int Np = Nq * Nq * Nq, Nfp = Nq * Nq;
@@ -266,6 +267,9 @@ k_gradient_mix(KParams P, MixParams MP, AffArrays A, ElemSet ES, const double *_
             gPhi[1] = gp[Np];
             gPhi[2] = gp[2 * Np];
         }
+        if (Qcopy)  // as in k_gradient_aff
+#pragma unroll
+            for (int s = 0; s < 5; ++s) __builtin_nontemporal_store(q[s], Qcopy + (int64_t)Np * (s + 5 * e) + n);
         const ThermoD t = thermo_d(P, q, Phi);
         grad_arg_f<SMAG>(P, MP, q, t, buoy, G);
         thv = SMAG ? G[4] : 1.0f;
