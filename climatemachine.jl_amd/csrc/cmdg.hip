@@ -82,7 +82,7 @@ struct cmdg_ctx {
     KParams P;
     KArrays A;
     hipStream_t stream;
-    double *d_vg = nullptr, *d_sg = nullptr, *d_D = nullptr, *d_aux = nullptr, *d_gf = nullptr, *d_Qs = nullptr;
+    double *d_vg = nullptr, *d_sg = nullptr, *d_D = nullptr, *d_aux = nullptr, *d_gf = nullptr, *d_Qs = nullptr, *d_Qt = nullptr;
     int32_t *d_nbr = nullptr, *d_bnd = nullptr;
     // affine-brick specialisation (see cmdg_affine.h)
     bool affine = false;
@@ -275,7 +275,7 @@ int launch_rhs(cmdg_ctx *c, const double *Q, double *tend, double alpha, double 
 
 int launch_copy(cmdg_ctx *c, double *dst, const double *src, int64_t n) {
     TimedLaunch tl(c, KIND_COPY);
-    hipLaunchKernelGGL(k_copy, dim3(2048), dim3(256), 0, c->stream, dst, src, n);
+    hipLaunchKernelGGL(k_copy, dim3((unsigned)std::min<int64_t>(2048, (n + 255) / 256)), dim3(256), 0, c->stream, dst, src, n);
     return check_hip(c, hipGetLastError(), "copy launch");
 }
 
@@ -675,6 +675,14 @@ int create_impl(const cmdg_desc *d, const cmdg_brick *brick, void *stream, cmdg_
     if (d->precision != CMDG_MIXED && (rc = upload<double>(c, &c->d_gf, nullptr, (size_t)Np * c->ngf * E)))
         return rc;
     if ((rc = upload<double>(c, &c->d_Qs, nullptr, (size_t)Np * 5 * E))) return rc;
+    // a third state buffer for odd step counts (cmdg_lsrk54_steps), up to 1 GiB and where
+    // there is room (CMDG_THIRD_STATE_BUFFER=0: never): without it such a call copies the state
+    const char *qenv = std::getenv("CMDG_THIRD_STATE_BUFFER");
+    if (!(qenv && qenv[0] == '0') && (size_t)Np * 5 * E * sizeof(double) <= (size_t)1 << 30 &&
+        hipMalloc((void **)&c->d_Qt, (size_t)Np * 5 * E * sizeof(double)) != hipSuccess) {
+        c->d_Qt = nullptr;
+        (void)hipGetLastError();
+    }
     if (c->d_gf &&
         (rc = check_hip(c, hipMemset(c->d_gf, 0, (size_t)Np * c->ngf * E * sizeof(double)), "hipMemset")))
         return rc;
@@ -722,7 +730,7 @@ int create_impl(const cmdg_desc *d, const cmdg_brick *brick, void *stream, cmdg_
                 }
             const char *tenv = std::getenv("CMDG_NEIGHBOUR_STATIC_TRACE");  // 1: always read it
             c->AA.aux_cont = (cont && !(tenv && tenv[0] == '1')) ? 1 : 0;
-            if ((rc = upload(c, &c->d_str, st.data(), st.size()))) return rc;
+            if (!c->AA.aux_cont && (rc = upload(c, &c->d_str, st.data(), st.size()))) return rc;
             // the FP64 viscosity planes (mixed contexts carry the stress form instead)
             const int nnu = viscosity_planes(c->smag, P.a_gPhi >= 0);
             if (d->precision != CMDG_MIXED && nnu > 0 &&
@@ -892,6 +900,7 @@ int cmdg_destroy(cmdg_ctx *c) {
     (void)hipFree(c->d_aux);
     (void)hipFree(c->d_gf);
     (void)hipFree(c->d_Qs);
+    (void)hipFree(c->d_Qt);
     (void)hipFree(c->d_geo);
     (void)hipFree(c->d_nbe);
     (void)hipFree(c->d_W);
@@ -948,22 +957,20 @@ int cmdg_lsrk54_steps(cmdg_ctx *c, double *Q, double *dQ, double t, double dt, i
     // Every stage reads its neighbours' volume state, so it writes the next stage's
     // state to another buffer: the stages alternate between the caller's Q (C) and the
     // context buffer S, and no caller code runs between the steps of one call.  Over
-    // 5 nsteps stages the result lands in C when that count is even; when it is odd,
-    // S <- C first and the first stage reads S.  A diffusive context's first gradient pass
-    // reads C and writes the copy as it goes: 40 B a node and no launch, where a copy moves 80.
-    // One step, us, copy kernel / fused: FP64 25^3 1100 / 1095, 33^3 2702 / 2675, 48^3 8125 /
-    // 8048; mixed 16^3 277 / 275, 25^3 851 / 854, 30^3 1484 / 1493, 33^3 2085 / 2057, 64^3
-    // 15139 / 14885.  The mixed passes lose to those stores where the two states fit the
-    // last-level cache but not the L2s, 64 to 160 MiB a state: there the copy kernel stays.
-    const int64_t bytes = (int64_t)c->Np * 5 * c->nelem * (int64_t)sizeof(double), MiB = 1 << 20;
-    const bool fused_copy = c->diffusive && !(c->mixed && bytes > 64 * MiB && bytes <= 160 * MiB);
-    double *C = Q, *S = c->d_Qs;
+    // 5 nsteps stages the result lands in C when that count is even.  When it is odd, the
+    // first three stages go C -> S -> T -> C through a third buffer.  A context whose state is
+    // too large for one (create_impl) copies instead: S <- C first and the first stage reads
+    // S; a diffusive context's first gradient pass reads C and writes that copy as it goes.
+    // One step, us, copy kernel / copy in the gradient pass / third buffer: FP64 33^3 2702 /
+    // 2675 / 2648, 25^3 1100 / 1095 / 1082; mixed 25^3 with gravity 956 / 961 / 933, 33^3 2085 /
+    // 2057 / 2031, 64^3 15139 / 14885 / -; Euler 128 elements 40.1 / - / 38.0.
+    double *C = Q, *S = c->d_Qs, *T = c->d_Qt;
     double *src = C, *dst = S;
-    const bool odd = (nsteps % 2) != 0;
-    if (odd) {
+    const bool odd = (nsteps % 2) != 0, copied = odd && !T;
+    if (copied) {
         src = S;
         dst = C;
-        if (!fused_copy && (rc = launch_copy(c, S, C, (int64_t)c->Np * 5 * c->nelem))) return rc;
+        if (!c->diffusive && (rc = launch_copy(c, S, C, (int64_t)c->Np * 5 * c->nelem))) return rc;
     }
     for (int64_t step = 0; step < nsteps; ++step)
         for (int s = 0; s < 5; ++s) {
@@ -980,14 +987,16 @@ int cmdg_lsrk54_steps(cmdg_ctx *c, double *Q, double *dQ, double t, double dt, i
             const double dq_read = (s == 0 && step > 0) ? 0.0 : 1.0;
             const int dq_store = !(s == 4 && step < nsteps - 1);
             if (c->diffusive) {
-                const bool first = odd && fused_copy && step == 0 && s == 0;
+                const bool first = copied && step == 0 && s == 0;
                 if ((rc = launch_gradient(c, first ? C : src, first ? S : nullptr, wa))) return rc;
             }
             if ((rc = launch_tendency(c, src, dQ, 1.0, dq_read, 1, dst, a, bdt, c->diffusive ? 0 : wa, dq_store)))
                 return rc;
-            double *tmp = src;
+            // the buffer after next: S or C in turn, T once in the first step of an odd count
+            double *next = src;
+            if (odd && T && step == 0 && s < 3) next = s == 0 ? T : s == 1 ? C : S;
             src = dst;
-            dst = tmp;
+            dst = next;
         }
     return CMDG_OK;
 }
