@@ -95,6 +95,7 @@ struct cmdg_ctx {
     double *d_sa = nullptr;    // static fields by class
     int32_t *d_order = nullptr;  // tiled traversal order of the affine launches (null: none)
     const int32_t *ord_grad = nullptr, *ord_tend = nullptr;  // per pass: d_order or null (storage)
+    bool wide = false;  // face tasks in waves of their own (small meshes)
     // mixed precision (FP32 fluxes and gradient flux)
     bool mixed = false;
     MixParams MP{};
@@ -172,10 +173,20 @@ int launch_gradient_impl(cmdg_ctx *c, const double *Q, double *Qcopy, int write_
     // N^2 (Smagorinsky-Lilly) needs theta_v only under a gravitational potential
     const bool buoy = c->P.a_gPhi >= 0;
 #define CMDG_GRAD_MIX(SMAG, LEARN, BUOY)                                                                       \
-    hipLaunchKernelGGL((k_gradient_mix<Nq, SMAG, LEARN, BUOY>), grid, block, 0, c->stream, c->P, c->MP, c->AA, ES, \
+    do {                                                                                                       \
+        if (c->wide) CMDG_GRAD_MIX_W(SMAG, LEARN, BUOY, true);                                                 \
+        else CMDG_GRAD_MIX_W(SMAG, LEARN, BUOY, false);                                                        \
+    } while (0)
+#define CMDG_GRAD_MIX_W(SMAG, LEARN, BUOY, W)                                                                  \
+    hipLaunchKernelGGL((k_gradient_mix<Nq, SMAG, LEARN, BUOY, W>), grid, dim3(block_threads<Nq, W>()), 0, c->stream, c->P, c->MP, c->AA, ES, \
                        Q, c->d_aux, c->d_gf32, Qcopy, write_aux, c->d_mlp)
 #define CMDG_GRAD_AFF(SMAG, BUOY)                                                                               \
-    hipLaunchKernelGGL((k_gradient_aff<Nq, SMAG, BUOY>), grid, block, 0, c->stream, c->P, c->AA, ES, Q, c->d_aux, \
+    do {                                                                                                        \
+        if (c->wide) CMDG_GRAD_AFF_W(SMAG, BUOY, true);                                                         \
+        else CMDG_GRAD_AFF_W(SMAG, BUOY, false);                                                                \
+    } while (0)
+#define CMDG_GRAD_AFF_W(SMAG, BUOY, W)                                                                          \
+    hipLaunchKernelGGL((k_gradient_aff<Nq, SMAG, BUOY, W>), grid, dim3(block_threads<Nq, W>()), 0, c->stream, c->P, c->AA, ES, Q, c->d_aux, \
                        c->d_gf, c->d_nu, Qcopy, write_aux)
     if (c->mixed) {
         if (c->learned) {
@@ -198,6 +209,8 @@ int launch_gradient_impl(cmdg_ctx *c, const double *Q, double *Qcopy, int write_
         hipLaunchKernelGGL((k_gradient<Nq, false>), grid, block, 0, c->stream, c->P, c->A, Q, c->d_aux, c->d_gf, Qcopy, write_aux);
 #undef CMDG_GRAD_MIX
 #undef CMDG_GRAD_AFF
+#undef CMDG_GRAD_AFF_W
+#undef CMDG_GRAD_MIX_W
     return check_hip(c, hipGetLastError(), "gradient launch");
 }
 
@@ -208,10 +221,20 @@ int launch_tendency_impl(cmdg_ctx *c, const double *Q, double *tend, double alph
     dim3 grid((unsigned)xcd_grid(c->affine ? ES.count : c->nelem)), block(NT);
     TimedLaunch tl(c, KIND_TENDENCY);
 #define CMDG_TEND_MIX(DIFF, ISO, MODE)                                                                           \
-    hipLaunchKernelGGL((k_tendency_mix<Nq, DIFF, ISO, MODE>), grid, block, 0, c->stream, c->P, c->MP, c->AA, ES, Q, \
+    do {                                                                                                          \
+        if (c->wide) CMDG_TEND_MIX_W(DIFF, ISO, MODE, true);                                                      \
+        else CMDG_TEND_MIX_W(DIFF, ISO, MODE, false);                                                             \
+    } while (0)
+#define CMDG_TEND_MIX_W(DIFF, ISO, MODE, W)                                                                       \
+    hipLaunchKernelGGL((k_tendency_mix<Nq, DIFF, ISO, MODE, W>), grid, dim3(block_threads<Nq, W>()), 0, c->stream, c->P, c->MP, c->AA, ES, Q, \
                        c->d_gf32, c->d_aux, tend, alpha, beta, Qout, rka, bdt, write_aux, dq_store)
 #define CMDG_TEND_AFF(DIFF, NNU, MODE)                                                                            \
-    hipLaunchKernelGGL((k_tendency_aff<Nq, DIFF, NNU, MODE>), grid, block, 0, c->stream, c->P, c->AA, ES, Q,      \
+    do {                                                                                                          \
+        if (c->wide) CMDG_TEND_AFF_W(DIFF, NNU, MODE, true);                                                      \
+        else CMDG_TEND_AFF_W(DIFF, NNU, MODE, false);                                                             \
+    } while (0)
+#define CMDG_TEND_AFF_W(DIFF, NNU, MODE, W)                                                                       \
+    hipLaunchKernelGGL((k_tendency_aff<Nq, DIFF, NNU, MODE, W>), grid, dim3(block_threads<Nq, W>()), 0, c->stream, c->P, c->AA, ES, Q,      \
                        c->d_gf, c->d_nu, c->d_aux, tend, alpha, beta, Qout, rka, bdt, write_aux, dq_store)
 #define CMDG_TEND(DIFF, SMAG, MODE)                                                                               \
     do {                                                                                                          \
@@ -237,6 +260,8 @@ int launch_tendency_impl(cmdg_ctx *c, const double *Q, double *tend, double alph
 #undef CMDG_TEND
 #undef CMDG_TEND_MIX
 #undef CMDG_TEND_AFF
+#undef CMDG_TEND_AFF_W
+#undef CMDG_TEND_MIX_W
     return check_hip(c, hipGetLastError(), "tendency launch");
 }
 
@@ -766,6 +791,15 @@ int create_impl(const cmdg_desc *d, const cmdg_brick *brick, void *stream, cmdg_
             } else {
                 crep.clear();
             }
+            // Wide blocks (face tasks in waves of their own, beside the volume waves) where the
+            // mesh leaves the chip idle: up to 3 elements a CU at N = 4 and 6 at N = 3, all in
+            // flight at once.  Without / with, us a pass: N = 4 FP64 128 elements 38 / 32 (Euler
+            // step), 162 / 135 (2 LES steps), 512 176 / 158, 768 234 / 226 and 272 / 273, 1024
+            // 214 / 259; mixed 128 142 / 122, 768 203 / 186, 1024 195 / 182 and 107 / 117; N = 3
+            // 1536 225 / 214, 271 / 267, 277 / 251, 2048 243 / 267, 310 / 296.
+            // (CMDG_WIDE_BLOCKS=0 or 1 chooses.)
+            const char *wenv = std::getenv("CMDG_WIDE_BLOCKS");
+            c->wide = wenv ? wenv[0] == '1' : E <= (Nq == 5 ? 768 : 1536);
             // tiled traversal.  CMDG_ELEMENT_TILE=T sets cubic tiles of edge T (0 keeps
             // the storage order) and "TX,TY,TZ" tile extents along x, y, z (0: the whole
             // axis); CMDG_TILED_PASSES = tendency, gradient, both or none chooses the passes

@@ -83,6 +83,13 @@ template <int Nq> __device__ __forceinline__ int face_node(int f, int fn) {
 // 3), each task's result goes to LDS, and each node then adds the results of its
 // faces in face order (the reference's order).
 
+// On a mesh too small to fill the chip (WIDE) a block has waves of their own for the face
+// tasks, one lane a task, which run beside the volume waves instead of after them.
+template <int Nq> constexpr int face_threads() { return (6 * Nq * Nq + 63) / 64 * 64; }
+template <int Nq, bool WIDE> constexpr int block_threads() {
+    return threads_for<Nq>() + (WIDE ? face_threads<Nq>() : 0);
+}
+
 // A static auxiliary field (Phi, p_ref) at volume node vn of element e, or dflt when
 // the model has no such field.
 template <int Nq>
@@ -100,7 +107,9 @@ __device__ __forceinline__ double own_aux(const KParams &P, const double *__rest
 // fills row d of the gradient only, so four values carry the whole jump of the gradient
 // flux: u_c and h_tot here, and with a gravitational potential the fifth, N^2's
 // (row d of grad theta_v . grad Phi / theta_v); jump_gradient_flux spreads them.
-template <int Nq, bool SMAG, bool BUOY>
+// OWN: the element's own gradient argument is formed here from its state (the operations of
+// its volume lanes, so their bits) instead of read from sG.
+template <int Nq, bool SMAG, bool BUOY, bool OWN>
 __device__ __forceinline__ void face_gradient_aff(const KParams &P, const AffArrays &A, int64_t e, int f, int fn,
                                                   int32_t ne, const double *__restrict__ Q,
                                                   const double (*sG)[Nq * Nq * Nq], double jump[5]) {
@@ -109,9 +118,16 @@ __device__ __forceinline__ void face_gradient_aff(const KParams &P, const AffArr
     const int d = f >> 1, vn = face_node<Nq>(f, fn);
     const double nd = (f & 1) ? 1.0 : -1.0;
     const int64_t ce = static_class(A, e);
-    double G[5], Gp[5], Gs[5];
+    double G[5], Gp[5], Gs[5], qm[5];
+    if (OWN) {
 #pragma unroll
-    for (int s = 0; s < 5; ++s) G[s] = (s < 4 || buoy) ? sG[s][vn] : 0.0;
+        for (int s = 0; s < 5; ++s) qm[s] = Q[(int64_t)Np * (s + 5 * e) + vn];
+        const Thermo t = thermo(P, qm, own_aux<Nq>(P, A.sa, ce, vn, P.a_Phi, -0.0));
+        grad_arg<buoy>(P, qm, t, buoy ? theta_v(P, t) : 0.0, G);
+    } else {
+#pragma unroll
+        for (int s = 0; s < 5; ++s) G[s] = (s < 4 || buoy) ? sG[s][vn] : 0.0;
+    }
     if (ne >= 0) {
         const int fo = f ^ 1;
         // the neighbour's state at the shared node, from its volume (the gradient pass
@@ -184,11 +200,11 @@ constexpr int viscosity_planes(bool smag, bool buoy) { return smag ? (buoy ? 3 :
 // tendency 1005 -> 1017), 25^3 with gravity 120 -> 106 (151 -> 151), 33^3 constant
 // viscosity 242 -> 199 (338 -> 366).  Register caps of 96 and 80 spill (15 and 37
 // registers) and cost 763 and 1173 us at 48^3.
-template <int Nq, bool SMAG, bool BUOY>
-__global__ void __launch_bounds__(threads_for<Nq>())
+template <int Nq, bool SMAG, bool BUOY, bool WIDE>
+__global__ void __launch_bounds__((block_threads<Nq, WIDE>()))
 k_gradient_aff(KParams P, AffArrays A, ElemSet ES, const double *__restrict__ Q, double *__restrict__ aux,
                double *__restrict__ gfo, double *__restrict__ nuo, double *__restrict__ Qcopy, int write_aux) {
-    constexpr int Np = Nq * Nq * Nq, Nfp = Nq * Nq, NT = threads_for<Nq>();
+    constexpr int Np = Nq * Nq * Nq, Nfp = Nq * Nq, NV = threads_for<Nq>();
     constexpr bool buoy = SMAG && BUOY;
     constexpr int NG = buoy ? 5 : 4, NGF = SMAG ? 10 : 9, NNU = viscosity_planes(SMAG, BUOY);
     __shared__ double sD[Nq * Nq];
@@ -229,13 +245,24 @@ k_gradient_aff(KParams P, AffArrays A, ElemSet ES, const double *__restrict__ Q,
 #pragma unroll
         for (int s = 0; s < NG; ++s) sG[s][n] = G[s];
     }
-    __syncthreads();
-    // lifted central jumps of all face nodes, spread over every lane
-    for (int t = n; t < 6 * Nfp; t += NT) {
-        double J[5];
-        face_gradient_aff<Nq, SMAG, BUOY>(P, A, e, t / Nfp, t % Nfp, nb[t / Nfp], Q, sG, J);
+    // lifted central jumps of all face nodes, spread over every lane (WIDE: over the face
+    // waves, meanwhile)
+    if (WIDE) {
+        const int t = n - NV;
+        if (t >= 0 && t < 6 * Nfp) {
+            double J[5];
+            face_gradient_aff<Nq, SMAG, BUOY, true>(P, A, e, t / Nfp, t % Nfp, A.nbe[6 * e + t / Nfp], Q, sG, J);
 #pragma unroll
-        for (int s = 0; s < NG; ++s) sJ[s][t] = J[s];
+            for (int s = 0; s < NG; ++s) sJ[s][t] = J[s];
+        }
+    } else {
+        __syncthreads();
+        for (int t = n; t < 6 * Nfp; t += NV) {
+            double J[5];
+            face_gradient_aff<Nq, SMAG, BUOY, false>(P, A, e, t / Nfp, t % Nfp, nb[t / Nfp], Q, sG, J);
+#pragma unroll
+            for (int s = 0; s < NG; ++s) sJ[s][t] = J[s];
+        }
     }
     __syncthreads();
 
@@ -301,9 +328,11 @@ k_gradient_aff(KParams P, AffArrays A, ElemSet ES, const double *__restrict__ Q,
 // The neighbour's second-order row is formed here from its gradient flux and viscosity at
 // the shared node (the strain-rate row, d h_tot / d x_d, nu_d; WithDivergence the two other
 // diagonal entries): the operations, and so the bits, of the neighbour's own row.
-template <int Nq, bool DIFF, int NNU>
-__device__ __forceinline__ void face_flux_aff(const KParams &P, const AffArrays &A, int64_t ce, int f, int fn,
-                                              int32_t ne, const double (*sQ)[Nq * Nq * Nq], const double *__restrict__ Q,
+// OWN: the element's own side is read from memory and its second-order row formed here too
+// (its volume lanes' bits again); otherwise its state is staged in sQ and the row is f2own.
+template <int Nq, bool DIFF, int NNU, bool OWN>
+__device__ __forceinline__ void face_flux_aff(const KParams &P, const AffArrays &A, int64_t e, int64_t ce, int f,
+                                              int fn, int32_t ne, const double (*sQ)[Nq * Nq * Nq], const double *__restrict__ Q,
                                               const double *__restrict__ gfi, const double *__restrict__ nui,
                                               const double *f2own, double flux[5]) {
     constexpr bool SMAG = NNU > 0;
@@ -314,11 +343,10 @@ __device__ __forceinline__ void face_flux_aff(const KParams &P, const AffArrays 
     const double h = nd * 0.5;
     const bool wall = ne < 0;
     const int fo = f ^ 1;
-    // the own state at the face's volume node, staged in LDS; the neighbour's from its
-    // volume
+    // the own state at the face's volume node; the neighbour's from its volume
     double q[5], qp[5];
 #pragma unroll
-    for (int s = 0; s < 5; ++s) q[s] = sQ[s][vn];
+    for (int s = 0; s < 5; ++s) q[s] = OWN ? Q[(int64_t)Np * (s + 5 * e) + vn] : sQ[s][vn];
     const double Phi = own_aux<Nq>(P, A.sa, ce, vn, P.a_Phi, -0.0);
     const double ref_p = own_aux<Nq>(P, A.sa, ce, vn, P.a_ref_p, 0.0);
     double Php = Phi, refpp = ref_p;
@@ -358,8 +386,19 @@ __device__ __forceinline__ void face_flux_aff(const KParams &P, const AffArrays 
             nud = nu[0];
         }
         flux2_row_parts<SMAG>(P, qp, S0, S1, S2, trS, nud, gd, d, F2p);
+        double F2m[5];
+        if (OWN) {
+            const double *gm = gfi + (int64_t)Np * NGF * e + vn;
+            const double g0[1] = {0.0}, gP[3] = {0.0, 0.0, 0.0};
+            double nu[3];
+            if (SMAG) nu[0] = nui[(int64_t)Np * (NNU * e + (NNU == 3 ? d : 0)) + vn];
+            else viscosity<false>(P, q[0], g0, gP, 0.0, nu);
+            const double tr = !SMAG && P.with_div ? (gm[Np * 3] + gm[Np * 6]) + gm[Np * 8] : 0.0;
+            flux2_row_parts<SMAG>(P, q, gm[Np * pick3(d, 3, 4, 5)], gm[Np * pick3(d, 4, 6, 7)],
+                                  gm[Np * pick3(d, 5, 7, 8)], tr, nu[0], gm[Np * d], d, F2m);
+        }
 #pragma unroll
-        for (int v = 0; v < TR_F2; ++v) f2[v] = (f2own[v] + F2p[1 + v]) * h;
+        for (int v = 0; v < TR_F2; ++v) f2[v] = ((OWN ? F2m[1 + v] : f2own[v]) + F2p[1 + v]) * h;
     }
     __builtin_amdgcn_sched_barrier(0);
     const Thermo tm = thermo(P, q, Phi);
@@ -405,13 +444,14 @@ __device__ __forceinline__ void face_flux_aff(const KParams &P, const AffArrays 
 // tasks first, both sides read from memory instead of LDS, cut the missed lines to 213 B and
 // cost 1069 us: the added vector-memory instructions weigh more.
 // At Nq = 4 five waves spill.
-template <int Nq, bool DIFF, int NNU, int MODE>
-__global__ void __launch_bounds__(threads_for<Nq>()) __attribute__((amdgpu_waves_per_eu(Nq == 5 ? 5 : 4)))
+template <int Nq, bool DIFF, int NNU, int MODE, bool WIDE>
+__global__ void __launch_bounds__((block_threads<Nq, WIDE>()))
+__attribute__((amdgpu_waves_per_eu(WIDE ? 1 : Nq == 5 ? 5 : 4)))
 k_tendency_aff(KParams P, AffArrays A, ElemSet ES, const double *__restrict__ Q,
                const double *__restrict__ gfi, const double *__restrict__ nui, double *__restrict__ aux,
                double *__restrict__ tend, double alpha, double beta, double *__restrict__ Qout, double rka,
                double bdt, int write_aux, int dq_store) {
-    constexpr int Np = Nq * Nq * Nq, Nfp = Nq * Nq, NT = threads_for<Nq>();
+    constexpr int Np = Nq * Nq * Nq, Nfp = Nq * Nq, NV = threads_for<Nq>();
     constexpr bool SMAG = NNU > 0;
     constexpr int NGF = SMAG ? 10 : 9;
     __shared__ double sD[Nq * Nq];
@@ -434,6 +474,16 @@ k_tendency_aff(KParams P, AffArrays A, ElemSet ES, const double *__restrict__ Q,
 
     const int64_t ce = static_class(A, e);
     double q[5], gf[9], u[3], nu[3], Fv[5], MI = 0.0;
+    if (WIDE) {
+        const int t = n - NV;
+        if (t >= 0 && t < 6 * Nfp) {
+            double fl5[5];
+            face_flux_aff<Nq, DIFF, NNU, true>(P, A, e, ce, t / Nfp, t % Nfp, A.nbe[6 * e + t / Nfp], nullptr, Q, gfi,
+                                               nui, nullptr, fl5);
+#pragma unroll
+            for (int s = 0; s < 5; ++s) sFl[t][s] = fl5[s];
+        }
+    }
     if (act) {
         const double *qb = Q + (int64_t)Np * 5 * e + n;
 #pragma unroll
@@ -473,7 +523,7 @@ k_tendency_aff(KParams P, AffArrays A, ElemSet ES, const double *__restrict__ Q,
                 flux2_row<SMAG>(P, q, gf, nu, ax, F2);
                 int fn;
                 const int f = node_face_dir<Nq>(i, j, k, ax, fn);
-                if (f >= 0)
+                if (!WIDE && f >= 0)
 #pragma unroll
                     for (int v = 0; v < TR_F2; ++v) sFl[f * Nfp + fn][v] = F2[1 + v];
 #pragma unroll
@@ -542,16 +592,18 @@ k_tendency_aff(KParams P, AffArrays A, ElemSet ES, const double *__restrict__ Q,
         }
     }
     // numerical fluxes of all face nodes, spread over every lane
-    for (int t = n; t < 6 * Nfp; t += NT) {
-        double own[TR_F2], fl5[5];
-        if (DIFF)
+    if (!WIDE) {
+        for (int t = n; t < 6 * Nfp; t += NV) {
+            double own[TR_F2], fl5[5];
+            if (DIFF)
 #pragma unroll
-            for (int v = 0; v < TR_F2; ++v) own[v] = sFl[t][v];
-        face_flux_aff<Nq, DIFF, NNU>(P, A, ce, t / Nfp, t % Nfp, nb[t / Nfp], sQ, Q, gfi, nui, own, fl5);
+                for (int v = 0; v < TR_F2; ++v) own[v] = sFl[t][v];
+            face_flux_aff<Nq, DIFF, NNU, false>(P, A, e, ce, t / Nfp, t % Nfp, nb[t / Nfp], sQ, Q, gfi, nui, own, fl5);
 #pragma unroll
-        for (int s = 0; s < 5; ++s) sFl[t][s] = fl5[s];
+            for (int s = 0; s < 5; ++s) sFl[t][s] = fl5[s];
+        }
+        __syncthreads();
     }
-    __syncthreads();
 
     if (act) {
         // the face fluxes of this node's faces, in face order

@@ -225,8 +225,10 @@ __device__ __forceinline__ void grad_arg_f(const KParams &P, const MixParams &M,
 // BUOY: the context has a gravitational potential (FlatOrientation), so Smagorinsky-Lilly's
 // N^2 = grad theta_v . grad Phi / theta_v needs theta_v and its gradient; without one
 // (grad Phi = 0, N^2 = 0 exactly) the kernel evaluates neither.
-template <int Nq, bool SMAG, bool LEARN, bool BUOY>
-__global__ void __launch_bounds__(threads_for<Nq>()) __attribute__((amdgpu_waves_per_eu(Nq == 5 ? 7 : 5)))
+// WIDE: as for k_gradient_aff, the face waves form the own side's argument themselves.
+template <int Nq, bool SMAG, bool LEARN, bool BUOY, bool WIDE>
+__global__ void __launch_bounds__((block_threads<Nq, WIDE>()))
+__attribute__((amdgpu_waves_per_eu(WIDE ? 1 : Nq == 5 ? 7 : 5)))
 k_gradient_mix(KParams P, MixParams MP, AffArrays A, ElemSet ES, const double *__restrict__ Q,
                double *__restrict__ aux, float *__restrict__ gfo, double *__restrict__ Qcopy, int write_aux,
                const MlpDev *__restrict__ mlp) {
@@ -281,15 +283,23 @@ k_gradient_mix(KParams P, MixParams MP, AffArrays A, ElemSet ES, const double *_
 #pragma unroll
         for (int s = 0; s < NG; ++s) sG[s][n] = G[s];
     }
-    __syncthreads();
-    // lifted central jumps n (G* - G-) of all face nodes, spread over every lane
-    for (int t = n; t < 6 * Nfp; t += NT) {
+    if (!WIDE) __syncthreads();
+    // lifted central jumps n (G* - G-) of all face nodes, spread over every lane (WIDE: over
+    // the face waves, before the barrier)
+    for (int t = WIDE ? (n >= NT ? n - NT : 6 * Nfp) : n; t < 6 * Nfp; t += WIDE ? 6 * Nfp : NT) {
         const int f = t / Nfp, fn = t % Nfp, d = f >> 1, vn = face_node<Nq>(f, fn);
         const float nd = (f & 1) ? 1.0f : -1.0f;
-        const int32_t ne = nb[f];
+        const int32_t ne = WIDE ? A.nbe[6 * e + f] : nb[f];
         float Gm[5], Gp[5];
+        if (WIDE) {
+            double qm[5];
 #pragma unroll
-        for (int s = 0; s < 5; ++s) Gm[s] = s < NG ? sG[s][vn] : 0.0f;
+            for (int s = 0; s < 5; ++s) qm[s] = Q[(int64_t)Np * (s + 5 * e) + vn];
+            grad_arg_f<SMAG>(P, MP, qm, thermo_d(P, qm, own_aux<Nq>(P, A.sa, ce, vn, P.a_Phi, -0.0)), buoy, Gm);
+        } else {
+#pragma unroll
+            for (int s = 0; s < 5; ++s) Gm[s] = s < NG ? sG[s][vn] : 0.0f;
+        }
         float jump[5];
         if (ne >= 0) {
             const int fo = f ^ 1;
@@ -358,7 +368,7 @@ k_gradient_mix(KParams P, MixParams MP, AffArrays A, ElemSet ES, const double *_
         }
         grad_flux_f<SMAG, buoy>(g, gPhi, thv, gf);
     }
-    if (LEARN) {
+    if (LEARN && (!WIDE || n < NT)) {
         // the network runs on the assembled gradient (volume + lifted face jumps):
         // it is nonlinear, so it cannot be split over the two contributions
         float x[MLP_IN];
@@ -379,6 +389,32 @@ k_gradient_mix(KParams P, MixParams MP, AffArrays A, ElemSet ES, const double *_
 }
 
 // ------------------------------------------------------------------ tendency (mixed)
+// The own side of a face along axis d from the FP64 state q and the stress form at gb: the
+// operations of k_tendency_mix's volume phase (no contraction), so its bits.
+template <int Nq, bool DIFF, bool ISO>
+__device__ __forceinline__ void own_rows_mix(const KParams &P, const MixParams &MP, const float *gb, const double q[5],
+                                             double Phi, double ref_p, double p_e, int d, float own[9]) {
+    constexpr int Np = Nq * Nq * Nq;
+    using L = StressForm<ISO>;
+    const ThermoD t = thermo_d(P, q, Phi);
+    float qf[5], F[5];
+#pragma unroll
+    for (int s = 0; s < 5; ++s) qf[s] = (float)q[s];
+    const float ri = 1.0f / qf[0];
+    const float uf[3] = {qf[1] * ri, qf[2] * ri, qf[3] * ri};
+    flux1_row_f(qf, uf, (float)t.p, (float)(MP.ref_sub ? t.p - ref_p : t.p - p_e), d, F);
+#pragma unroll
+    for (int s = 1; s < 5; ++s) own[s - 1] = F[s];
+    own[8] = fabsf(pick3(d, uf[0], uf[1], uf[2])) + (MP.rusanov ? sqrtf(MP.gammaR * (float)t.temp) : 0.0f);
+    if (DIFF) {
+        const float tau[3] = {gb[Np * L::tau(d, 0)], gb[Np * L::tau(d, 1)], gb[Np * L::tau(d, 2)]};
+        float F2[5];
+        flux2_row_stress(tau, gb[Np * (L::E + d)], qf, F2);
+#pragma unroll
+        for (int v = 0; v < TR_F2; ++v) own[4 + v] = F2[1 + v];
+    }
+}
+
 // Numerical flux at face node fn of face f of element e.  The own side arrives
 // precomputed by the volume phase (own[0..3]: entries 1-4 of the first-order flux row
 // along the face's axis, own[4..7]: the second-order row, own[8]: |u_d| + c; the row's
@@ -389,11 +425,12 @@ k_gradient_mix(KParams P, MixParams MP, AffArrays A, ElemSet ES, const double *_
 // its FP32-rounded state: the bits the neighbour's own volume phase forms for that row.
 // The jump q- - q+ is formed in FP64 from the own state, staged in LDS with Phi and
 // p_ref (sQ rows 0-4, 5, 6).
-template <int Nq, bool DIFF, bool ISO>
+// OWN: the own side is read from memory and own[] formed here (own_rows_mix).
+template <int Nq, bool DIFF, bool ISO, bool OWN>
 __device__ __forceinline__ void face_flux_mix(const KParams &P, const MixParams &MP, const AffArrays &A, int f, int fn,
-                                              int32_t ne, const double (*sQ)[Nq * Nq * Nq],
+                                              int64_t e, int64_t ce, int32_t ne, const double (*sQ)[Nq * Nq * Nq],
                                               const double *__restrict__ Q, const float *__restrict__ gfi,
-                                              const float own[9], double p_e, float flux[5]) {
+                                              float own[9], double p_e, float flux[5]) {
 #pragma clang fp contract(fast)
     constexpr int Np = Nq * Nq * Nq, Nfp = Nq * Nq;
     const int d = f >> 1, vn = face_node<Nq>(f, fn);
@@ -403,7 +440,9 @@ __device__ __forceinline__ void face_flux_mix(const KParams &P, const MixParams 
     double q[5], qp[5], Php, refpp;
     float t2p[3] = {0.0f, 0.0f, 0.0f}, e2p = 0.0f;  // the neighbour's stress-form row
 #pragma unroll
-    for (int s = 0; s < 5; ++s) q[s] = sQ[s][vn];
+    for (int s = 0; s < 5; ++s) q[s] = OWN ? Q[(int64_t)Np * (s + 5 * e) + vn] : sQ[s][vn];
+    const double Phim = OWN ? own_aux<Nq>(P, A.sa, ce, vn, P.a_Phi, -0.0) : sQ[5][vn];
+    const double refpm = OWN ? own_aux<Nq>(P, A.sa, ce, vn, P.a_ref_p, 0.0) : sQ[6][vn];
     if (!wall) {
         // the neighbour's state and stress-form row at the shared node, loaded together
         const double *qb = Q + (int64_t)Np * 5 * ne + face_node<Nq>(fo, fn);
@@ -417,8 +456,8 @@ __device__ __forceinline__ void face_flux_mix(const KParams &P, const MixParams 
             e2p = gn[Np * (L::E + d)];
         }
         if (A.aux_cont) {
-            Php = sQ[5][vn];
-            refpp = sQ[6][vn];
+            Php = Phim;
+            refpp = refpm;
         } else {
             Php = A.str[tri<Nfp>(ne, fo, 0, TR_S, fn)];
             refpp = A.str[tri<Nfp>(ne, fo, 1, TR_S, fn)];
@@ -429,9 +468,10 @@ __device__ __forceinline__ void face_flux_mix(const KParams &P, const MixParams 
 #pragma unroll
         for (int c = 0; c < 3; ++c)
             if (c == d) qp[1 + c] = -q[1 + c];  // reflect the normal momentum
-        Php = sQ[5][vn];
-        refpp = sQ[6][vn];
+        Php = Phim;
+        refpp = refpm;
     }
+    if (OWN) own_rows_mix<Nq, DIFF, ISO>(P, MP, gfi + (int64_t)Np * StressForm<ISO>::NGF * e + vn, q, Phim, refpm, p_e, d, own);
     const ThermoD tp = thermo_d(P, qp, Php);
     float qpf[5], upf[3], jump[5];
 #pragma unroll
@@ -471,8 +511,9 @@ __device__ __forceinline__ void face_flux_mix(const KParams &P, const MixParams 
 // nu_0) is already folded into it.
 // Six waves per SIMD at Nq = 5: the register cap this asks for (80) spills nothing there
 // (at Nq = 4 it would, so that order keeps the compiler's choice).
-template <int Nq, bool DIFF, bool ISO, int MODE>
-__global__ void __launch_bounds__(threads_for<Nq>()) __attribute__((amdgpu_waves_per_eu(Nq == 5 ? 6 : 1)))
+template <int Nq, bool DIFF, bool ISO, int MODE, bool WIDE>
+__global__ void __launch_bounds__((block_threads<Nq, WIDE>()))
+__attribute__((amdgpu_waves_per_eu(!WIDE && Nq == 5 ? 6 : 1)))
 k_tendency_mix(KParams P, MixParams MP, AffArrays A, ElemSet ES, const double *__restrict__ Q,
                const float *__restrict__ gfi, double *__restrict__ aux, double *__restrict__ tend, double alpha,
                double beta, double *__restrict__ Qout, double rka, double bdt, int write_aux, int dq_store) {
@@ -509,6 +550,16 @@ k_tendency_mix(KParams P, MixParams MP, AffArrays A, ElemSet ES, const double *_
         const double qe[5] = {q0[0], q0[Np], q0[2 * Np], q0[3 * Np], q0[4 * Np]};
         const double Phe = P.a_Phi >= 0 ? A.sa[(int64_t)Np * P.naux * ce + (int64_t)Np * P.a_Phi] : -0.0;
         p_e = thermo_d(P, qe, Phe).p;
+    }
+    if (WIDE && n >= NT) {
+        const int t = n - NT;
+        if (t < 6 * Nfp) {
+            float own[9], fl5[5];
+            face_flux_mix<Nq, DIFF, ISO, true>(P, MP, A, t / Nfp, t % Nfp, e, ce, A.nbe[6 * e + t / Nfp], nullptr, Q, gfi,
+                                               own, p_e, fl5);
+#pragma unroll
+            for (int s = 0; s < 5; ++s) sFc[t][s] = fl5[s];
+        }
     }
     float qf[5], uf[3], sf[L::NREAD], gPhi[3] = {0.0f, 0.0f, 0.0f}, pf = 0.0f, pmf = 0.0f, cm = 0.0f, drho = 0.0f;
     float MI = 0.0f;
@@ -556,7 +607,7 @@ k_tendency_mix(KParams P, MixParams MP, AffArrays A, ElemSet ES, const double *_
             flux1_row_f(qf, uf, pf, pmf, ax, F);
             int fn;
             const int f = node_face_dir<Nq>(i, j, k, ax, fn);
-            if (f >= 0) {
+            if (!WIDE && f >= 0) {
 #pragma unroll
                 for (int s = 1; s < 5; ++s) sFc[f * Nfp + fn][s - 1] = F[s];
                 sFc[f * Nfp + fn][8] = fabsf(uf[ax]) + cm;
@@ -564,7 +615,7 @@ k_tendency_mix(KParams P, MixParams MP, AffArrays A, ElemSet ES, const double *_
             if (DIFF) {
                 const float t[3] = {sf[L::tau(ax, 0)], sf[L::tau(ax, 1)], sf[L::tau(ax, 2)]};
                 flux2_row_stress(t, sf[L::E + ax], qf, F2);
-                if (f >= 0)
+                if (!WIDE && f >= 0)
 #pragma unroll
                     for (int v = 0; v < TR_F2; ++v) sFc[f * Nfp + fn][4 + v] = F2[1 + v];
 #pragma unroll
@@ -606,13 +657,13 @@ k_tendency_mix(KParams P, MixParams MP, AffArrays A, ElemSet ES, const double *_
         sQ[5][n] = Phi;
         sQ[6][n] = ref_p;
     }
-    __syncthreads();
+    if (!WIDE) __syncthreads();
     // numerical fluxes of all face nodes, spread over every lane
-    for (int t = n; t < 6 * Nfp; t += NT) {
+    for (int t = WIDE ? 6 * Nfp : n; t < 6 * Nfp; t += NT) {
         float own[9], fl5[5];
 #pragma unroll
         for (int c = 0; c < 9; ++c) own[c] = sFc[t][c];
-        face_flux_mix<Nq, DIFF, ISO>(P, MP, A, t / Nfp, t % Nfp, nb[t / Nfp], sQ, Q, gfi, own, p_e, fl5);
+        face_flux_mix<Nq, DIFF, ISO, false>(P, MP, A, t / Nfp, t % Nfp, e, ce, nb[t / Nfp], sQ, Q, gfi, own, p_e, fl5);
 #pragma unroll
         for (int s = 0; s < 5; ++s) sFc[t][s] = fl5[s];
     }
@@ -626,7 +677,7 @@ k_tendency_mix(KParams P, MixParams MP, AffArrays A, ElemSet ES, const double *_
     if (MODE == 1 && act && beta != 0.0)
 #pragma unroll
         for (int s = 0; s < 5; ++s) dq[s] = __builtin_nontemporal_load(tb + Np * s);
-    __syncthreads();
+    if (!WIDE) __syncthreads();
 
     if (act) {
 #pragma unroll
