@@ -38,8 +38,8 @@
 #include "../../include/cmdg.h"
 
 #include "cmdg_physics.h"
-#include "cmdg_general.h"
 #include "cmdg_affine.h"
+#include "cmdg_general.h"
 #include "cmdg_mixed.h"
 #include "cmdg_learn.h"
 #include "cmdg_diag.h"
@@ -89,7 +89,8 @@ struct cmdg_ctx {
     AffArrays AA{};
     double *d_geo = nullptr, *d_W = nullptr, *d_Wf = nullptr;
     int32_t *d_nbe = nullptr;
-    double *d_nu = nullptr;    // FP64 path: viscosity planes (Smagorinsky-Lilly)
+    double *d_nu = nullptr;    // FP64 path: viscosity planes (Smagorinsky-Lilly), nnu of them
+    int nnu = 0;
     double *d_str = nullptr;   // static face trace
     int32_t *d_cls = nullptr;  // static-field class of each element (null: none)
     double *d_sa = nullptr;    // static fields by class
@@ -188,6 +189,14 @@ int launch_gradient_impl(cmdg_ctx *c, const double *Q, double *Qcopy, int write_
 #define CMDG_GRAD_AFF_W(SMAG, BUOY, W)                                                                          \
     hipLaunchKernelGGL((k_gradient_aff<Nq, SMAG, BUOY, W>), grid, dim3(block_threads<Nq, W>()), 0, c->stream, c->P, c->AA, ES, Q, c->d_aux, \
                        c->d_gf, c->d_nu, Qcopy, write_aux)
+#define CMDG_GRAD_GEN(SMAG, BUOY)                                                                                \
+    do {                                                                                                        \
+        if (c->wide) CMDG_GRAD_GEN_W(SMAG, BUOY, true);                                                         \
+        else CMDG_GRAD_GEN_W(SMAG, BUOY, false);                                                                \
+    } while (0)
+#define CMDG_GRAD_GEN_W(SMAG, BUOY, W)                                                                          \
+    hipLaunchKernelGGL((k_gradient<Nq, SMAG, BUOY, W>), grid, dim3(block_threads<Nq, W>()), 0, c->stream, c->P, \
+                       c->A, Q, c->d_aux, c->d_gf, c->d_nu, Qcopy, write_aux)
     if (c->mixed) {
         if (c->learned) {
             if (buoy) CMDG_GRAD_MIX(true, true, true);
@@ -203,10 +212,13 @@ int launch_gradient_impl(cmdg_ctx *c, const double *Q, double *Qcopy, int write_
             else CMDG_GRAD_AFF(true, false);
         } else
             CMDG_GRAD_AFF(false, false);
-    } else if (c->smag)
-        hipLaunchKernelGGL((k_gradient<Nq, true>), grid, block, 0, c->stream, c->P, c->A, Q, c->d_aux, c->d_gf, Qcopy, write_aux);
-    else
-        hipLaunchKernelGGL((k_gradient<Nq, false>), grid, block, 0, c->stream, c->P, c->A, Q, c->d_aux, c->d_gf, Qcopy, write_aux);
+    } else if (c->smag) {
+        if (c->P.a_gPhi >= 0) CMDG_GRAD_GEN(true, true);
+        else CMDG_GRAD_GEN(true, false);
+    } else
+        CMDG_GRAD_GEN(false, false);
+#undef CMDG_GRAD_GEN
+#undef CMDG_GRAD_GEN_W
 #undef CMDG_GRAD_MIX
 #undef CMDG_GRAD_AFF
 #undef CMDG_GRAD_AFF_W
@@ -244,10 +256,16 @@ int launch_tendency_impl(cmdg_ctx *c, const double *Q, double *tend, double alph
         } else if (c->affine) {                                                                                   \
             if (c->P.a_gPhi >= 0) CMDG_TEND_AFF(DIFF, viscosity_planes(SMAG, true), MODE);                        \
             else CMDG_TEND_AFF(DIFF, viscosity_planes(SMAG, false), MODE);                                        \
-        } else                                                                                                    \
-            hipLaunchKernelGGL((k_tendency<Nq, DIFF, SMAG, MODE>), grid, block, 0, c->stream, c->P, c->A, Q,      \
-                               c->d_gf, c->d_aux, tend, alpha, beta, Qout, rka, bdt, write_aux, dq_store);       \
+        } else if (c->wide) {                                                                                     \
+            CMDG_TEND_GEN(DIFF, SMAG, MODE, true);                                                                \
+        } else {                                                                                                  \
+            CMDG_TEND_GEN(DIFF, SMAG, MODE, false);                                                               \
+        }                                                                                                         \
     } while (0)
+#define CMDG_TEND_GEN(DIFF, SMAG, MODE, W)                                                                        \
+    hipLaunchKernelGGL((k_tendency<Nq, DIFF, SMAG, MODE, W>), grid, dim3(block_threads<Nq, W>()), 0, c->stream,   \
+                       c->P, c->A, Q, c->d_gf, c->d_nu, c->nnu, c->d_aux, tend, alpha, beta, Qout, rka, bdt,      \
+                       write_aux, dq_store)
     if (mode == 0) {
         if (!c->diffusive) CMDG_TEND(false, false, 0);
         else if (c->smag) CMDG_TEND(true, true, 0);
@@ -262,6 +280,7 @@ int launch_tendency_impl(cmdg_ctx *c, const double *Q, double *tend, double alph
 #undef CMDG_TEND_AFF
 #undef CMDG_TEND_AFF_W
 #undef CMDG_TEND_MIX_W
+#undef CMDG_TEND_GEN
     return check_hip(c, hipGetLastError(), "tendency launch");
 }
 
@@ -711,6 +730,11 @@ int create_impl(const cmdg_desc *d, const cmdg_brick *brick, void *stream, cmdg_
     if (c->d_gf &&
         (rc = check_hip(c, hipMemset(c->d_gf, 0, (size_t)Np * c->ngf * E * sizeof(double)), "hipMemset")))
         return rc;
+    // the FP64 viscosity planes (mixed contexts carry the stress form instead)
+    c->nnu = viscosity_planes(c->smag, P.a_gPhi >= 0);
+    if (d->precision != CMDG_MIXED && c->nnu > 0 &&
+        (rc = upload<double>(c, &c->d_nu, nullptr, (size_t)Np * c->nnu * E)))
+        return rc;
     c->A.D = c->d_D;
     c->A.nelem = E;
     std::vector<int64_t> crep;  // first element of each static-field class (empty: no classes)
@@ -756,11 +780,6 @@ int create_impl(const cmdg_desc *d, const cmdg_brick *brick, void *stream, cmdg_
             const char *tenv = std::getenv("CMDG_NEIGHBOUR_STATIC_TRACE");  // 1: always read it
             c->AA.aux_cont = (cont && !(tenv && tenv[0] == '1')) ? 1 : 0;
             if (!c->AA.aux_cont && (rc = upload(c, &c->d_str, st.data(), st.size()))) return rc;
-            // the FP64 viscosity planes (mixed contexts carry the stress form instead)
-            const int nnu = viscosity_planes(c->smag, P.a_gPhi >= 0);
-            if (d->precision != CMDG_MIXED && nnu > 0 &&
-                (rc = upload<double>(c, &c->d_nu, nullptr, (size_t)Np * nnu * E)))
-                return rc;
             c->AA.geo = c->d_geo;
             c->AA.nbe = c->d_nbe;
             c->AA.W = c->d_W;
@@ -791,15 +810,6 @@ int create_impl(const cmdg_desc *d, const cmdg_brick *brick, void *stream, cmdg_
             } else {
                 crep.clear();
             }
-            // Wide blocks (face tasks in waves of their own, beside the volume waves) where the
-            // mesh leaves the chip idle: up to 3 elements a CU at N = 4 and 6 at N = 3, all in
-            // flight at once.  Without / with, us a pass: N = 4 FP64 128 elements 38 / 32 (Euler
-            // step), 162 / 135 (2 LES steps), 512 176 / 158, 768 234 / 226 and 272 / 273, 1024
-            // 214 / 259; mixed 128 142 / 122, 768 203 / 186, 1024 195 / 182 and 107 / 117; N = 3
-            // 1536 225 / 214, 271 / 267, 277 / 251, 2048 243 / 267, 310 / 296.
-            // (CMDG_WIDE_BLOCKS=0 or 1 chooses.)
-            const char *wenv = std::getenv("CMDG_WIDE_BLOCKS");
-            c->wide = wenv ? wenv[0] == '1' : E <= (Nq == 5 ? 768 : 1536);
             // tiled traversal.  CMDG_ELEMENT_TILE=T sets cubic tiles of edge T (0 keeps
             // the storage order) and "TX,TY,TZ" tile extents along x, y, z (0: the whole
             // axis); CMDG_TILED_PASSES = tendency, gradient, both or none chooses the passes
@@ -852,6 +862,18 @@ int create_impl(const cmdg_desc *d, const cmdg_brick *brick, void *stream, cmdg_
             }
         }
     }
+    // Wide blocks (face tasks in waves of their own, beside the volume waves) where the
+    // mesh leaves the chip idle: up to 3 elements a CU at N = 4 and 6 at N = 3, all in
+    // flight at once.  Without / with, us a pass: N = 4 FP64 128 elements 38 / 32 (Euler
+    // step), 162 / 135 (2 LES steps), 512 176 / 158, 768 234 / 226 and 272 / 273, 1024
+    // 214 / 259; mixed 128 142 / 122, 768 203 / 186, 1024 195 / 182 and 107 / 117; N = 3
+    // 1536 225 / 214, 271 / 267, 277 / 251, 2048 243 / 267, 310 / 296.  The general kernels'
+    // line at N = 4 lies a block a CU lower (their tasks hold more registers): 256 170 / 136,
+    // 512 214 / 184 and 245 / 229 with gravity, 768 236 / 252 and 285 / 311; N = 3 1536 232 /
+    // 214 and 281 / 264, 2744 334 / 332 and 409 / 425.
+    // (CMDG_WIDE_BLOCKS=0 or 1 chooses.)
+    const char *wenv = std::getenv("CMDG_WIDE_BLOCKS");
+    c->wide = wenv ? wenv[0] == '1' : E <= (Nq != 5 ? 1536 : c->affine ? 768 : 512);
     if (!c->affine) {
         // general meshes: per-node geometry xi (9), M, MI, the face geometry and the
         // neighbour node of every face node (affine bricks read none of these)

@@ -1,29 +1,103 @@
 // cmdg_general.h -- DG kernels for general (curvilinear) hexahedral meshes: per-node
 // metric terms, per-face-node normals and surface weights, vmap+ gathers.
+//
+// As in the brick kernels (cmdg_affine.h) the 6 Nfp face nodes of an element are tasks of
+// their own, whose results reach the node lanes through LDS in the reference's face order, and
+// on a small mesh (WIDE) the tasks have waves of their own.  On the node lanes a face node's
+// up to three faces ran one after the other in both waves, with the fluxes of the whole volume
+// phase held in registers (166 and 182 in the tendency and the gradient, now 126 and 94).
+// The same operations in the same order, so the same bits.
+// Bound by memory on a large mesh (per-node metric terms and per-face-node normals: about 250
+// B a node in the gradient, 390 in the tendency), by the chain of dependent reads (neighbour
+// index, its state and gradient flux) on one that fits the chip at once.  us a pass, gradient
+// + tendency, before -> now: 24^3 Smagorinsky-Lilly 128 + 286 -> 100 + 214, with gravity 135 +
+// 312 -> 138 + 261 (a task's theta_v costs what the faces' order gave), 14^3 27.8 + 52.6 ->
+// 22.8 + 42.7, N = 3 24^3 69 + 132 -> 58 + 102.  A neighbour index read one task ahead
+// lengthens the registers' lives by more than it hides (14 x 12 x 10 viscous right-hand side
+// 35.7 against 36.9 us with it).
 #pragma once
-#include "cmdg_physics.h"
+#include "cmdg_affine.h"
 
 namespace cmdg {
 
 // ------------------------------------------------------------------ gradient kernel
-template <int Nq, bool SMAG>
-__global__ void __launch_bounds__(threads_for<Nq>())
+// Lifted jump M^-1 Mf (Phi(G*) - Phi(n G-)) of face node fn of face f of element e,
+// CentralNumericalFluxGradient.
+// OWN as in face_gradient_aff.
+template <int Nq, bool BUOY, bool OWN>
+__device__ __forceinline__ void face_gradient(const KParams &P, const KArrays &A, const double *__restrict__ Q,
+                                              const double *__restrict__ aux, int64_t e, int f, int fn,
+                                              const double (*sG)[Nq * Nq * Nq], double *jump) {
+    constexpr int Np = Nq * Nq * Nq, Nfp = Nq * Nq, NGF = BUOY ? 10 : 9;
+    const int64_t idx = fn + (int64_t)Nfp * (f + 6 * e);
+    const double *sgp = A.sg + 5 * idx;
+    const double nv[3] = {sgp[0], sgp[1], sgp[2]};
+    const double sM = sgp[3], vMI = sgp[4];
+    const int vn = face_node<Nq>(f, fn);
+    const bool wall = A.bnd[f + 6 * e] != 0;
+    const int32_t nb = wall ? (int32_t)(e * Np + vn) : A.nbr[idx];
+    const int64_t ep = nb / Np;
+    const int vp = nb - (int)ep * Np;
+    double qp[5], Gm[5], Gp[5], Gs[3][5], nG[3][5];
+#pragma unroll
+    for (int s = 0; s < 5; ++s) qp[s] = Q[(int64_t)Np * (s + 5 * ep) + vp];
+    const double Php = P.a_Phi >= 0 ? aux[(int64_t)Np * (P.naux * ep + P.a_Phi) + vp] : -0.0;
+    const Aux a = load_aux(P, aux, Np, vn, e);
+    if (OWN) {
+        double q[5];
+#pragma unroll
+        for (int s = 0; s < 5; ++s) q[s] = Q[(int64_t)Np * (s + 5 * e) + vn];
+        const Thermo tm = thermo(P, q, a.Phi);
+        grad_arg<BUOY>(P, q, tm, BUOY ? theta_v(P, tm) : 0.0, Gm);
+    } else {
+#pragma unroll
+        for (int s = 0; s < 5; ++s) Gm[s] = (s < 4 || BUOY) ? sG[s][vn] : 0.0;
+    }
+    const double thv = Gm[4];
+    if (wall) {
+        double qb[5];
+        wall_state(qp, nv, 1.0, qb);
+#pragma unroll
+        for (int s = 0; s < 5; ++s) qp[s] = qb[s];
+    }
+    const Thermo tp = thermo(P, qp, Php);
+    grad_arg<BUOY>(P, qp, tp, BUOY ? theta_v(P, tp) : 0.0, Gp);
+#pragma unroll
+    for (int d = 0; d < 3; ++d)
+#pragma unroll
+        for (int s = 0; s < 5; ++s) {
+            Gs[d][s] = wall ? nv[d] * Gp[s] : nv[d] * (Gp[s] + Gm[s]) * 0.5;
+            nG[d][s] = nv[d] * Gm[s];
+        }
+    double gfs[10], gfm[10];
+    grad_flux<BUOY>(Gs, a, thv, gfs);
+    grad_flux<BUOY>(nG, a, thv, gfm);
+    const double w = vMI * sM;
+#pragma unroll
+    for (int s = 0; s < NGF; ++s) jump[s] = w * (gfs[s] - gfm[s]);
+}
+
+// nuo: viscosity planes (Np, viscosity_planes, nelem).  BUOY as in k_gradient_aff.
+template <int Nq, bool SMAG, bool BUOY, bool WIDE>
+__global__ void __launch_bounds__((block_threads<Nq, WIDE>()))
 k_gradient(KParams P, KArrays A, const double *__restrict__ Q, double *__restrict__ aux,
-           double *__restrict__ gfo, double *__restrict__ Qcopy, int write_aux) {
-    constexpr int Np = Nq * Nq * Nq, Nfp = Nq * Nq;
-    constexpr int NG = SMAG ? 5 : 4, NGF = SMAG ? 10 : 9;
+           double *__restrict__ gfo, double *__restrict__ nuo, double *__restrict__ Qcopy, int write_aux) {
+    constexpr int Np = Nq * Nq * Nq, Nfp = Nq * Nq, NV = threads_for<Nq>();
+    constexpr bool buoy = SMAG && BUOY;
+    constexpr int NG = buoy ? 5 : 4, NJ = buoy ? 10 : 9, NGF = SMAG ? 10 : 9, NNU = viscosity_planes(SMAG, BUOY);
     __shared__ double sD[Nq * Nq];
     __shared__ double sG[NG][Np];
+    __shared__ double sJ[NJ][6 * Nfp];
     const int64_t e = xcd_element(blockIdx.x, A.nelem);
     if (e >= A.nelem) return;
     const int n = threadIdx.x;
     if (n < Nq * Nq) sD[n] = A.D[n];
     const bool act = n < Np;
     const int i = n % Nq, j = (n / Nq) % Nq, k = n / (Nq * Nq);
-    double q[5], thv = 0.0;
+    double thv = 1.0, rho = 0.0;
     Aux a;
-    Thermo t;
     if (act) {
+        double q[5], G[5];
         const double *qb = Q + (int64_t)Np * 5 * e + n;
 #pragma unroll
         for (int s = 0; s < 5; ++s) q[s] = qb[Np * s];
@@ -32,18 +106,25 @@ k_gradient(KParams P, KArrays A, const double *__restrict__ Q, double *__restric
 #pragma unroll
             for (int s = 0; s < 5; ++s) qc[Np * s] = q[s];
         }
+        rho = q[0];
         a = load_aux(P, aux, Np, n, e);
-        t = thermo(P, q, a.Phi);
-        thv = theta_v(P, t);
+        const Thermo t = thermo(P, q, a.Phi);
+        if (buoy || (write_aux && P.a_theta_v >= 0)) thv = theta_v(P, t);
         if (write_aux) {
             double *ab = aux + (int64_t)Np * P.naux * e + n;
             if (P.a_theta_v >= 0) ab[(int64_t)Np * P.a_theta_v] = thv;
             if (P.a_air_T >= 0) ab[(int64_t)Np * P.a_air_T] = t.temp;
         }
-        double G[5];
-        grad_arg<SMAG>(P, q, t, thv, G);
+        grad_arg<buoy>(P, q, t, thv, G);
 #pragma unroll
         for (int s = 0; s < NG; ++s) sG[s][n] = G[s];
+    }
+    if (!WIDE) __syncthreads();
+    for (int t = WIDE ? (n >= NV ? n - NV : 6 * Nfp) : n; t < 6 * Nfp; t += WIDE ? 6 * Nfp : NV) {
+        double J[10];
+        face_gradient<Nq, buoy, WIDE>(P, A, Q, aux, e, t / Nfp, t % Nfp, sG, J);
+#pragma unroll
+        for (int s = 0; s < NJ; ++s) sJ[s][t] = J[s];
     }
     __syncthreads();
     if (!act) return;
@@ -81,109 +162,165 @@ k_gradient(KParams P, KArrays A, const double *__restrict__ Q, double *__restric
     }
 
     double gf[10], gfv[10];
-    grad_flux<SMAG>(gG, a, thv, gf);
-    grad_flux<SMAG>(gV, a, thv, gfv);
+    grad_flux<buoy>(gG, a, thv, gf);
+    grad_flux<buoy>(gV, a, thv, gfv);
 #pragma unroll
-    for (int s = 0; s < NGF; ++s) gf[s] += gfv[s];
+    for (int s = 0; s < NJ; ++s) gf[s] += gfv[s];
 
-    // lifted face jumps: M^-1 Mf (Phi(G*) - Phi(n G-)), CentralNumericalFluxGradient
-    double Gm[5];
-    grad_arg<SMAG>(P, q, t, thv, Gm);
+    // the lifted jumps of this node's faces, in face order
 #pragma unroll
     for (int dir = 0; dir < 3; ++dir) {
-        int fnd;
-        const int f = node_face_dir<Nq>(i, j, k, dir, fnd);
+        int fn;
+        const int f = node_face_dir<Nq>(i, j, k, dir, fn);
         if (f < 0) continue;
-        const int64_t idx = fnd + (int64_t)Nfp * (f + 6 * e);
-        const double *sgp = A.sg + 5 * idx;
-        double nv[3] = {sgp[0], sgp[1], sgp[2]};
-        const double sM = sgp[3], vMI = sgp[4];
-        double Gs[3][5], nG[3][5], Gp[5];
-        if (A.bnd[f + 6 * e] == 0) {
-            const int32_t nb = A.nbr[idx];
-            const int64_t ep = nb / Np;
-            const int vp = nb - (int)ep * Np;
-            double qp[5];
-            const double *qpb = Q + (int64_t)Np * 5 * ep + vp;
 #pragma unroll
-            for (int s = 0; s < 5; ++s) qp[s] = qpb[Np * s];
-            double Php = P.a_Phi >= 0 ? aux[(int64_t)Np * P.naux * ep + vp + (int64_t)Np * P.a_Phi] : -0.0;
-            Thermo tp = thermo(P, qp, Php);
-            double thp = SMAG ? theta_v(P, tp) : 0.0;
-            grad_arg<SMAG>(P, qp, tp, thp, Gp);
-#pragma unroll
-            for (int d = 0; d < 3; ++d)
-#pragma unroll
-                for (int s = 0; s < 5; ++s) Gs[d][s] = nv[d] * (Gp[s] + Gm[s]) * 0.5;
-        } else {
-            double qb[5];
-            wall_state(q, nv, 1.0, qb);
-            Thermo tb = thermo(P, qb, a.Phi);
-            double thb = SMAG ? theta_v(P, tb) : 0.0;
-            grad_arg<SMAG>(P, qb, tb, thb, Gp);
-#pragma unroll
-            for (int d = 0; d < 3; ++d)
-#pragma unroll
-                for (int s = 0; s < 5; ++s) Gs[d][s] = nv[d] * Gp[s];
-        }
-#pragma unroll
-        for (int d = 0; d < 3; ++d)
-#pragma unroll
-            for (int s = 0; s < 5; ++s) nG[d][s] = nv[d] * Gm[s];
-        double gfs[10], gfm[10];
-        grad_flux<SMAG>(Gs, a, thv, gfs);
-        grad_flux<SMAG>(nG, a, thv, gfm);
-        const double w = vMI * sM;
-#pragma unroll
-        for (int s = 0; s < NGF; ++s) gf[s] += w * (gfs[s] - gfm[s]);
+        for (int s = 0; s < NJ; ++s) gf[s] += sJ[s][f * Nfp + fn];
     }
     double *go = gfo + (int64_t)Np * NGF * e + n;
 #pragma unroll
-    for (int s = 0; s < NGF; ++s) go[Np * s] = gf[s];
+    for (int s = 0; s < NJ; ++s) go[Np * s] = gf[s];
+    if (SMAG) {
+        if (!buoy && write_aux) go[Np * 9] = 0.0;  // N^2
+        double nu[3];
+        viscosity<SMAG, BUOY>(P, rho, gf, a.gPhi, a.Delta, nu);
+        double *no = nuo + (int64_t)Np * NNU * e + n;
+#pragma unroll
+        for (int s = 0; s < NNU; ++s) no[Np * s] = nu[s];
+    }
 }
 
 // ------------------------------------------------------------------ tendency kernel
+// One side of a face or one node: its fluxes from the state, static fields and gradient flux.
+template <int Nq, bool DIFF, bool SMAG>
+__device__ __forceinline__ void node_flux2(const KParams &P, const double *__restrict__ gfi,
+                                           const double *__restrict__ nui, int nnu, int64_t e, int n,
+                                           const double q[5], double F2[3][5]) {
+    constexpr int Np = Nq * Nq * Nq, NGF = SMAG ? 10 : 9;
+    double gf[9], nu[3];
+    const double *gb = gfi + (int64_t)Np * NGF * e + n;
+#pragma unroll
+    for (int s = 0; s < 9; ++s) gf[s] = gb[Np * s];
+    if (SMAG) {
+        const double *nb = nui + (int64_t)Np * nnu * e + n;
+#pragma unroll
+        for (int d = 0; d < 3; ++d) nu[d] = nb[Np * (nnu == 3 ? d : 0)];
+    } else {
+        const double gP[3] = {0.0, 0.0, 0.0};
+        viscosity<false>(P, q[0], gf, gP, 0.0, nu);
+    }
+#pragma unroll
+    for (int d = 0; d < 3; ++d) flux2_row<SMAG>(P, q, gf, nu, d, F2[d]);
+}
+
+// Lifted numerical flux alpha M^-1 Mf F*.n of face node fn of face f of element e
+// (NumericalFluxes.jl:219-340, 670-715); alpha = 1 in MODE 1.
+template <int Nq, bool DIFF, bool SMAG, int MODE>
+__device__ __forceinline__ void face_flux(const KParams &P, const KArrays &A, const double *__restrict__ Q,
+                                          const double *__restrict__ gfi, const double *__restrict__ nui, int nnu,
+                                          const double *__restrict__ aux, int64_t e, int f, int fn, double alpha,
+                                          double out[5]) {
+    constexpr int Np = Nq * Nq * Nq, Nfp = Nq * Nq;
+    const int64_t idx = fn + (int64_t)Nfp * (f + 6 * e);
+    const double *sgp = A.sg + 5 * idx;
+    const double nv[3] = {sgp[0], sgp[1], sgp[2]};
+    const double w = (MODE == 0 ? alpha * sgp[4] : sgp[4]) * sgp[3];  // alpha * vMI * sM
+    const int vn = face_node<Nq>(f, fn);
+    const bool wall = A.bnd[f + 6 * e] != 0;
+    // at a wall the element itself stands in for the neighbour
+    const int32_t nb = wall ? (int32_t)(e * Np + vn) : A.nbr[idx];
+    const int64_t ep = nb / Np;
+    const int vp = nb - (int)ep * Np;
+    double q[5], qp[5];
+#pragma unroll
+    for (int s = 0; s < 5; ++s) {
+        q[s] = Q[(int64_t)Np * (s + 5 * e) + vn];
+        qp[s] = Q[(int64_t)Np * (s + 5 * ep) + vp];
+    }
+    const double h[3] = {nv[0] * 0.5, nv[1] * 0.5, nv[2] * 0.5};
+    double f2[5];
+    if (DIFF && !wall) {
+        double Fm[3][5], Fp[3][5];
+        node_flux2<Nq, DIFF, SMAG>(P, gfi, nui, nnu, e, vn, q, Fm);
+        node_flux2<Nq, DIFF, SMAG>(P, gfi, nui, nnu, ep, vp, qp, Fp);
+#pragma unroll
+        for (int s = 0; s < 5; ++s)
+            f2[s] = ((Fm[0][s] + Fp[0][s]) * h[0] + (Fm[1][s] + Fp[1][s]) * h[1]) + (Fm[2][s] + Fp[2][s]) * h[2];
+    }
+    __builtin_amdgcn_sched_barrier(0);  // the second-order part leaves five values
+    const double *am = aux + (int64_t)Np * P.naux * e + vn, *ap = aux + (int64_t)Np * P.naux * ep + vp;
+    const double Phim = P.a_Phi >= 0 ? am[(int64_t)Np * P.a_Phi] : -0.0, Phip = P.a_Phi >= 0 ? ap[(int64_t)Np * P.a_Phi] : -0.0;
+    const double refm = P.a_ref_p >= 0 ? am[(int64_t)Np * P.a_ref_p] : 0.0, refp = P.a_ref_p >= 0 ? ap[(int64_t)Np * P.a_ref_p] : 0.0;
+    if (wall) wall_state(q, nv, 2.0, qp);
+    const Thermo tm = thermo(P, q, Phim), tp = thermo(P, qp, Phip);
+    double Fm[3][5], Fp[3][5], flux[5];
+    flux1(P, q, tm.p, refm, Fm);
+    flux1(P, qp, tp.p, refp, Fp);
+#pragma unroll
+    for (int s = 0; s < 5; ++s)
+        flux[s] = -0.0 + (((Fm[0][s] + Fp[0][s]) * h[0] + (Fm[1][s] + Fp[1][s]) * h[1]) + (Fm[2][s] + Fp[2][s]) * h[2]);
+    if (P.rusanov) {
+        const double rim = 1.0 / q[0], rip = 1.0 / qp[0];
+        const double uNm = fabs((nv[0] * (rim * q[1]) + nv[1] * (rim * q[2])) + nv[2] * (rim * q[3]));
+        const double uNp = fabs((nv[0] * (rip * qp[1]) + nv[1] * (rip * qp[2])) + nv[2] * (rip * qp[3]));
+        const double mw = fmax(uNm + sqrt(P.gammaR * tm.temp), uNp + sqrt(P.gammaR * tp.temp));
+#pragma unroll
+        for (int s = 0; s < 5; ++s) flux[s] += (mw * (q[s] - qp[s])) * 0.5;
+    }
+    if (DIFF && !wall)
+#pragma unroll
+        for (int s = 0; s < 5; ++s) flux[s] += f2[s];
+#pragma unroll
+    for (int s = 0; s < 5; ++s) out[s] = w * flux[s];
+}
+
 // MODE 0: tend = alpha*RHS + beta*tend.   MODE 1: LSRK stage, tend is dQ:
 //   dQ <- RHS + dQ; Qout = Qin + bdt*dQ; dQ *= rka.  In MODE 1 beta = 0 says dQ holds
 //   zeros (the previous stage scaled it by rka = 0) and is not read; dq_store = 0 leaves
 //   the scaled dQ unstored (this stage's rka is 0 and the next stage gets beta = 0).
-template <int Nq, bool DIFF, bool SMAG, int MODE>
-__global__ void __launch_bounds__(threads_for<Nq>())
+template <int Nq, bool DIFF, bool SMAG, int MODE, bool WIDE>
+__global__ void __launch_bounds__((block_threads<Nq, WIDE>()))
 k_tendency(KParams P, KArrays A, const double *__restrict__ Q, const double *__restrict__ gfi,
-           double *__restrict__ aux, double *__restrict__ tend, double alpha, double beta,
-           double *__restrict__ Qout, double rka, double bdt, int write_aux, int dq_store) {
-    constexpr int Np = Nq * Nq * Nq, Nfp = Nq * Nq;
-    constexpr int NGF = SMAG ? 10 : 9;
+           const double *__restrict__ nui, int nnu, double *__restrict__ aux, double *__restrict__ tend, double alpha,
+           double beta, double *__restrict__ Qout, double rka, double bdt, int write_aux, int dq_store) {
+    constexpr int Np = Nq * Nq * Nq, Nfp = Nq * Nq, NV = threads_for<Nq>();
     __shared__ double sD[Nq * Nq];
     __shared__ double sF[3][5][Np];
+    __shared__ double sFl[5][6 * Nfp];  // lifted face fluxes
     const int64_t e = xcd_element(blockIdx.x, A.nelem);
     if (e >= A.nelem) return;
     const int n = threadIdx.x;
     if (n < Nq * Nq) sD[n] = A.D[n];
     const bool act = n < Np;
     const int i = n % Nq, j = (n / Nq) % Nq, k = n / (Nq * Nq);
+    for (int t = WIDE ? (n >= NV ? n - NV : 6 * Nfp) : n; t < 6 * Nfp; t += WIDE ? 6 * Nfp : NV) {
+        double fl5[5];
+        face_flux<Nq, DIFF, SMAG, MODE>(P, A, Q, gfi, nui, nnu, aux, e, t / Nfp, t % Nfp, alpha, fl5);
+#pragma unroll
+        for (int s = 0; s < 5; ++s) sFl[s][t] = fl5[s];
+    }
 
-    double q[5], gf[10], F1[3][5], F2[3][5], src[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-    Aux a;
-    Thermo t;
+    double q[5], src[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
     double MI = 0.0;
     if (act) {
         const double *qb = Q + (int64_t)Np * 5 * e + n;
 #pragma unroll
         for (int s = 0; s < 5; ++s) q[s] = qb[Np * s];
-        a = load_aux(P, aux, Np, n, e);
-        t = thermo(P, q, a.Phi);
+        const Aux a = load_aux(P, aux, Np, n, e);
+        const Thermo t = thermo(P, q, a.Phi);
         if (write_aux) {
             double *ab = aux + (int64_t)Np * P.naux * e + n;
             if (P.a_theta_v >= 0) ab[(int64_t)Np * P.a_theta_v] = theta_v(P, t);
             if (P.a_air_T >= 0) ab[(int64_t)Np * P.a_air_T] = t.temp;
         }
-        flux1(P, q, t.p, a.ref_p, F1);
+        double F[3][5];
+        flux1(P, q, t.p, a.ref_p, F);
         if (DIFF) {
-            const double *gb = gfi + (int64_t)Np * NGF * e + n;
+            double F2[3][5];
+            node_flux2<Nq, DIFF, SMAG>(P, gfi, nui, nnu, e, n, q, F2);
 #pragma unroll
-            for (int s = 0; s < NGF; ++s) gf[s] = gb[Np * s];
-            flux2<SMAG>(P, q, gf, a, F2);
+            for (int d = 0; d < 3; ++d)
+#pragma unroll
+                for (int s = 0; s < 5; ++s) F[d][s] += F2[d][s];
         }
         const double *vg = A.vg + (int64_t)Np * NVG * e + n;
         const double M = vg[Np * 9];
@@ -192,11 +329,7 @@ k_tendency(KParams P, KArrays A, const double *__restrict__ Q, const double *__r
         for (int ax = 0; ax < 3; ++ax) {
             const double x1 = vg[Np * ax], x2 = vg[Np * (ax + 3)], x3 = vg[Np * (ax + 6)];
 #pragma unroll
-            for (int s = 0; s < 5; ++s) {
-                double Fx = F1[0][s], Fy = F1[1][s], Fz = F1[2][s];
-                if (DIFF) { Fx += F2[0][s]; Fy += F2[1][s]; Fz += F2[2][s]; }
-                sF[ax][s][n] = M * ((x1 * Fx + x2 * Fy) + x3 * Fz);
-            }
+            for (int s = 0; s < 5; ++s) sF[ax][s][n] = M * ((x1 * F[0][s] + x2 * F[1][s]) + x3 * F[2][s]);
         }
         if (P.gravity) {
             // Gravity() source (tendencies_momentum.jl:60-72)
@@ -232,68 +365,14 @@ k_tendency(KParams P, KArrays A, const double *__restrict__ Q, const double *__r
         T[s] = (MODE == 0 ? alpha * tv : tv) + out;
     }
 
-    // face fluxes of the faces this node lies on (NumericalFluxes.jl:219-340, 670-715)
-    const bool on_face = i == 0 || i == Nq - 1 || j == 0 || j == Nq - 1 || k == 0 || k == Nq - 1;
-    double csm = 0.0;
-    if (on_face && P.rusanov) csm = sqrt(P.gammaR * t.temp);
+    // the face fluxes of this node's faces, in face order
 #pragma unroll
     for (int dir = 0; dir < 3; ++dir) {
-        int fnd;
-        const int f = node_face_dir<Nq>(i, j, k, dir, fnd);
+        int fn;
+        const int f = node_face_dir<Nq>(i, j, k, dir, fn);
         if (f < 0) continue;
-        const int64_t idx = fnd + (int64_t)Nfp * (f + 6 * e);
-        const double *sgp = A.sg + 5 * idx;
-        const double nv[3] = {sgp[0], sgp[1], sgp[2]};
-        const double w = (MODE == 0 ? alpha * sgp[4] : sgp[4]) * sgp[3];  // alpha * vMI * sM
-        const bool wall = A.bnd[f + 6 * e] != 0;
-        double qp[5], Fp[3][5], Phip, refpp;
-        Aux ap;
-        if (!wall) {
-            const int32_t nb = A.nbr[idx];
-            const int64_t ep = nb / Np;
-            const int vp = nb - (int)ep * Np;
-            const double *qpb = Q + (int64_t)Np * 5 * ep + vp;
 #pragma unroll
-            for (int s = 0; s < 5; ++s) qp[s] = qpb[Np * s];
-            ap = load_aux(P, aux, Np, vp, ep);
-            Phip = ap.Phi;
-            refpp = ap.ref_p;
-        } else {
-            wall_state(q, nv, 2.0, qp);
-            ap = a;
-            Phip = a.Phi;
-            refpp = a.ref_p;
-        }
-        Thermo tp = thermo(P, qp, Phip);
-        flux1(P, qp, tp.p, refpp, Fp);
-        const double h[3] = {nv[0] * 0.5, nv[1] * 0.5, nv[2] * 0.5};
-        double flux[5];
-#pragma unroll
-        for (int s = 0; s < 5; ++s)
-            flux[s] = -0.0 + (((F1[0][s] + Fp[0][s]) * h[0] + (F1[1][s] + Fp[1][s]) * h[1]) + (F1[2][s] + Fp[2][s]) * h[2]);
-        if (P.rusanov) {
-            const double rim = 1.0 / q[0], rip = 1.0 / qp[0];
-            const double uNm = fabs((nv[0] * (rim * q[1]) + nv[1] * (rim * q[2])) + nv[2] * (rim * q[3]));
-            const double uNp = fabs((nv[0] * (rip * qp[1]) + nv[1] * (rip * qp[2])) + nv[2] * (rip * qp[3]));
-            const double mw = fmax(uNm + csm, uNp + sqrt(P.gammaR * tp.temp));
-#pragma unroll
-            for (int s = 0; s < 5; ++s) flux[s] += (mw * (q[s] - qp[s])) * 0.5;
-        }
-        if (DIFF && !wall) {
-            const int32_t nb = A.nbr[idx];
-            const int64_t ep = nb / Np;
-            const int vp = nb - (int)ep * Np;
-            double gfp[10];
-            const double *gpb = gfi + (int64_t)Np * NGF * ep + vp;
-#pragma unroll
-            for (int s = 0; s < NGF; ++s) gfp[s] = gpb[Np * s];
-            flux2<SMAG>(P, qp, gfp, ap, Fp);
-#pragma unroll
-            for (int s = 0; s < 5; ++s)
-                flux[s] += ((F2[0][s] + Fp[0][s]) * h[0] + (F2[1][s] + Fp[1][s]) * h[1]) + (F2[2][s] + Fp[2][s]) * h[2];
-        }
-#pragma unroll
-        for (int s = 0; s < 5; ++s) T[s] -= w * flux[s];
+        for (int s = 0; s < 5; ++s) T[s] -= sFl[s][f * Nfp + fn];
     }
 
     if (MODE == 0) {

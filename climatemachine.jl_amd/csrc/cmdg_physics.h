@@ -146,7 +146,8 @@ __device__ __forceinline__ Aux load_aux(const KParams &P, const double *__restri
 // tendencies_energy.jl:7-21).
 __device__ __forceinline__ void flux1(const KParams &P, const double q[5], double p, double ref_p, double F[3][5]) {
     double pm = P.ref_sub ? (p - ref_p) : p;
-    double u[3] = {q[1] / q[0], q[2] / q[0], q[3] / q[0]};
+    const double rinv = 1.0 / q[0];
+    double u[3] = {div_by(q[1], q[0], rinv), div_by(q[2], q[0], rinv), div_by(q[3], q[0], rinv)};
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
         F[d][0] = q[1 + d];
@@ -158,57 +159,6 @@ __device__ __forceinline__ void flux1(const KParams &P, const double q[5], doubl
 
 // Julia eps(x) for x >= 0
 __device__ __forceinline__ double ulp_above(double x) { return nextafter(x, INFINITY) - x; }
-
-// Second-order flux: turbulence tensors (TurbulenceClosures.jl:366-404, 472-499) then
-// ViscousStress / ViscousFlux / DiffEnthalpyFlux (tendencies_momentum.jl:37-42,
-// tendencies_energy.jl:27-56).  gf = [grad h_tot (3), S (6), N2].
-template <bool SMAG>
-__device__ __forceinline__ void flux2(const KParams &P, const double q[5], const double *gf, const Aux &a, double F[3][5]) {
-    const double *S = gf + 3;
-    double Sm[3][3] = {{S[0], S[1], S[2]}, {S[1], S[3], S[4]}, {S[2], S[4], S[5]}};
-    double tau[3][3], Dt[3];
-    if (SMAG) {
-        double norm2 = ((((S[0] * S[0] + 2.0 * (S[1] * S[1])) + 2.0 * (S[2] * S[2])) + S[3] * S[3]) +
-                        2.0 * (S[4] * S[4])) + S[5] * S[5];
-        double normS = sqrt(2.0 * norm2);
-        double k[3] = {a.gPhi[0] / P.grav, a.gPhi[1] / P.grav, a.gPhi[2] / P.grav};
-        double Ri = gf[9] / (normS * normS + ulp_above(normS));
-        double fb2 = sqrt(fmin(fmax(1.0 - Ri * P.inv_Pr, 0.0), 1.0));
-        double CD = P.C_smag * a.Delta;
-        double nu0 = normS * (CD * CD) + 1e-5;
-        double dotk = (nu0 * k[0] + nu0 * k[1]) + nu0 * k[2];
-#pragma unroll
-        for (int d = 0; d < 3; ++d) {
-            double nuv = k[d] * dotk;
-            double nud = (nu0 - nuv) + nuv * fb2;
-            Dt[d] = nud * P.inv_Pr;
-#pragma unroll
-            for (int c = 0; c < 3; ++c) tau[d][c] = (-2.0 * nud) * Sm[d][c];
-        }
-    } else {
-        double nu = (P.turbulence == CMDG_CONSTANT_DYNAMIC_VISCOSITY) ? P.visc / q[0] : P.visc;
-        double trS = (Sm[0][0] + Sm[1][1]) + Sm[2][2];
-        double dv = ((2.0 * nu) / 3.0) * trS;
-#pragma unroll
-        for (int d = 0; d < 3; ++d) {
-            Dt[d] = nu * P.inv_Pr;
-#pragma unroll
-            for (int c = 0; c < 3; ++c) {
-                double v = (-2.0 * nu) * Sm[d][c];
-                if (P.with_div && d == c) v = v + dv;
-                tau[d][c] = v;
-            }
-        }
-    }
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-        F[d][0] = 0.0;
-#pragma unroll
-        for (int c = 0; c < 3; ++c) F[d][1 + c] = tau[d][c] * q[0];
-        double vf = (tau[d][0] * q[1] + tau[d][1] * q[2]) + tau[d][2] * q[3];
-        F[d][4] = vf + ((-Dt[d]) * gf[d]) * q[0];
-    }
-}
 
 // gradient argument G = (u, h_tot[, theta_v]) (AtmosModel.jl:622-690, energy.jl:20-31)
 template <bool SMAG>

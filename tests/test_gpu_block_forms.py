@@ -73,3 +73,13 @@ def test_state_buffers(variant, steps):
     env = {"CMDG_GENERAL_GEOMETRY": "1"} if form == "general" else {}
     prec = abi.MIXED if form == "mixed" else abi.FP64
     _same(_run(*case, prec, steps, **env), _run(*case, prec, steps, CMDG_THIRD_STATE_BUFFER="0", **env))
+
+
+@pytest.mark.parametrize("steps", [0, 2])
+@pytest.mark.parametrize("N", [3, 4])
+@pytest.mark.parametrize("name", CASES)
+def test_wide_blocks_general(name, N, steps):
+    case = _case(name, N)
+    env = {"CMDG_GENERAL_GEOMETRY": "1"}
+    _same(_run(*case, abi.FP64, steps, CMDG_WIDE_BLOCKS="0", **env),
+          _run(*case, abi.FP64, steps, CMDG_WIDE_BLOCKS="1", **env))
