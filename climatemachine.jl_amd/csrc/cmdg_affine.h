@@ -200,6 +200,13 @@ constexpr int viscosity_planes(bool smag, bool buoy) { return smag ? (buoy ? 3 :
 // tendency 1005 -> 1017), 25^3 with gravity 120 -> 106 (151 -> 151), 33^3 constant
 // viscosity 242 -> 199 (338 -> 366).  Register caps of 96 and 80 spill (15 and 37
 // registers) and cost 763 and 1173 us at 48^3.
+// The neighbours and the derivative matrix are read on every lane, not under a branch: its
+// end waits for what it read (and stored to LDS) before the state is even asked for, two
+// round trips a block.  In the tendency, likewise, every field of the node is asked for before
+// anything is waited for.  us, gradient + tendency: 48^3 Smagorinsky-Lilly 582 + 972 -> 554 +
+// 955, 33^3 constant viscosity 196 + 341 -> 183 + 334, 25^3 with gravity 107.8 + 147.9 ->
+// 104.5 + 146.5.  The face waves of a wide block read their own neighbour and fill the time
+// (128 elements the same or 1 us a step slower so), so there the matrix stays under its branch.
 template <int Nq, bool SMAG, bool BUOY, bool WIDE>
 __global__ void __launch_bounds__((block_threads<Nq, WIDE>()))
 k_gradient_aff(KParams P, AffArrays A, ElemSet ES, const double *__restrict__ Q, double *__restrict__ aux,
@@ -213,9 +220,15 @@ k_gradient_aff(KParams P, AffArrays A, ElemSet ES, const double *__restrict__ Q,
     const int64_t e = set_element(ES, blockIdx.x);
     if (e < 0) return;
     __shared__ int32_t nb[6];  // the element's face neighbours
-    if (threadIdx.x < 6) nb[threadIdx.x] = A.nbe[6 * e + threadIdx.x];
     const int n = threadIdx.x;
-    if (n < Nq * Nq) sD[n] = A.D[n];
+    int32_t nbn = 0;
+    double Dn = 0.0;
+    if (WIDE) {
+        if (n < Nq * Nq) sD[n] = A.D[n];
+    } else {  // on every lane (see above)
+        nbn = A.nbe[6 * e + min(n, 5)];
+        Dn = A.D[min(n, Nq * Nq - 1)];
+    }
     const bool act = n < Np;
     const int i = n % Nq, j = (n / Nq) % Nq, k = n / (Nq * Nq);
     const double *ge = A.geo + (int64_t)AFF_GEO * e;
@@ -245,6 +258,8 @@ k_gradient_aff(KParams P, AffArrays A, ElemSet ES, const double *__restrict__ Q,
 #pragma unroll
         for (int s = 0; s < NG; ++s) sG[s][n] = G[s];
     }
+    if (!WIDE && n < 6) nb[n] = nbn;
+    if (!WIDE && n < Nq * Nq) sD[n] = Dn;
     // lifted central jumps of all face nodes, spread over every lane (WIDE: over the face
     // waves, meanwhile)
     if (WIDE) {
@@ -465,9 +480,15 @@ k_tendency_aff(KParams P, AffArrays A, ElemSet ES, const double *__restrict__ Q,
     const int64_t e = set_element(ES, blockIdx.x);
     if (e < 0) return;
     __shared__ int32_t nb[6];  // the element's face neighbours
-    if (threadIdx.x < 6) nb[threadIdx.x] = A.nbe[6 * e + threadIdx.x];
     const int n = threadIdx.x;
-    if (n < Nq * Nq) sD[n] = A.D[n];
+    int32_t nbn = 0;
+    double Dn = 0.0;
+    if (WIDE) {
+        if (n < Nq * Nq) sD[n] = A.D[n];
+    } else {  // on every lane (see above)
+        nbn = A.nbe[6 * e + min(n, 5)];
+        Dn = A.D[min(n, Nq * Nq - 1)];
+    }
     const bool act = n < Np;
     const int i = n % Nq, j = (n / Nq) % Nq, k = n / (Nq * Nq);
     const double *ge = A.geo + (int64_t)AFF_GEO * e;
@@ -488,6 +509,19 @@ k_tendency_aff(KParams P, AffArrays A, ElemSet ES, const double *__restrict__ Q,
         const double *qb = Q + (int64_t)Np * 5 * e + n;
 #pragma unroll
         for (int s = 0; s < 5; ++s) q[s] = qb[Np * s];
+        // all of the node's fields before the first is waited for: the branch below would
+        // hold the rest back (WIDE: the other waves fill the time, the registers count more)
+        if (DIFF && !WIDE) {
+            const double *gb = gfi + (int64_t)Np * NGF * e + n;
+#pragma unroll
+            for (int s = 0; s < 9; ++s) gf[s] = gb[Np * s];
+            if (SMAG) {
+                const double *nb_ = nui + (int64_t)Np * NNU * e + n;
+#pragma unroll
+                for (int d = 0; d < 3; ++d) nu[d] = nb_[Np * (NNU == 3 ? d : 0)];
+            }
+        }
+        const double Wn = A.W[n];
         const Thermo t = thermo(P, q, own_aux<Nq>(P, A.sa, ce, n, P.a_Phi, -0.0));
         if (write_aux) {
             double *ab = aux + (int64_t)Np * P.naux * e + n;
@@ -500,7 +534,7 @@ k_tendency_aff(KParams P, AffArrays A, ElemSet ES, const double *__restrict__ Q,
         u[0] = div_by(q[1], q[0], rinv);
         u[1] = div_by(q[2], q[0], rinv);
         u[2] = div_by(q[3], q[0], rinv);
-        if (DIFF) {
+        if (DIFF && WIDE) {
             const double *gb = gfi + (int64_t)Np * NGF * e + n;
 #pragma unroll
             for (int s = 0; s < 9; ++s) gf[s] = gb[Np * s];
@@ -508,12 +542,13 @@ k_tendency_aff(KParams P, AffArrays A, ElemSet ES, const double *__restrict__ Q,
                 const double *nb_ = nui + (int64_t)Np * NNU * e + n;
 #pragma unroll
                 for (int d = 0; d < 3; ++d) nu[d] = nb_[Np * (NNU == 3 ? d : 0)];
-            } else {
-                const double gP[3] = {0.0, 0.0, 0.0};
-                viscosity<false>(P, q[0], gf, gP, 0.0, nu);
             }
         }
-        const double M = ge[3] * A.W[n];
+        if (DIFF && !SMAG) {
+            const double gP[3] = {0.0, 0.0, 0.0};
+            viscosity<false>(P, q[0], gf, gP, 0.0, nu);
+        }
+        const double M = ge[3] * Wn;
         MI = 1.0 / M;
 #pragma unroll
         for (int ax = 0; ax < 3; ++ax) {
@@ -538,6 +573,8 @@ k_tendency_aff(KParams P, AffArrays A, ElemSet ES, const double *__restrict__ Q,
             }
         }
     }
+    if (!WIDE && n < 6) nb[n] = nbn;
+    if (!WIDE && n < Nq * Nq) sD[n] = Dn;
     __syncthreads();
     // horizontal divergence of this node, into registers
     double T[5];

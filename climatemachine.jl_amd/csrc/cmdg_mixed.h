@@ -248,9 +248,10 @@ k_gradient_mix(KParams P, MixParams MP, AffArrays A, ElemSet ES, const double *_
     const int64_t ce = static_class(A, e);
     constexpr bool buoy = SMAG && BUOY;
     __shared__ int32_t nb[6];  // the element's face neighbours
-    if (threadIdx.x < 6) nb[threadIdx.x] = A.nbe[6 * e + threadIdx.x];
     const int n = threadIdx.x;
-    if (n < Nq * Nq) sD[n] = (float)A.D[n];
+    // on every lane, as in k_gradient_aff (64^3 learned 1145 -> 1124 us, N = 3 buoyant 19.7 -> 19.2)
+    const int32_t nbn = A.nbe[6 * e + min(n, 5)];
+    const double Dn = A.D[min(n, Nq * Nq - 1)];
     const bool act = n < Np;
     const int i = n % Nq, j = (n / Nq) % Nq, k = n / (Nq * Nq);
     const double *ge = A.geo + (int64_t)AFF_GEO * e;
@@ -283,6 +284,8 @@ k_gradient_mix(KParams P, MixParams MP, AffArrays A, ElemSet ES, const double *_
 #pragma unroll
         for (int s = 0; s < NG; ++s) sG[s][n] = G[s];
     }
+    if (n < 6) nb[n] = nbn;
+    if (n < Nq * Nq) sD[n] = (float)Dn;
     if (!WIDE) __syncthreads();
     // lifted central jumps n (G* - G-) of all face nodes, spread over every lane (WIDE: over
     // the face waves, before the barrier)
@@ -511,6 +514,11 @@ __device__ __forceinline__ void face_flux_mix(const KParams &P, const MixParams 
 // nu_0) is already folded into it.
 // Six waves per SIMD at Nq = 5: the register cap this asks for (80) spills nothing there
 // (at Nq = 4 it would, so that order keeps the compiler's choice).
+// EARLY: neighbours and derivative matrix on every lane, as in k_gradient_aff: 23 x 19 x 17
+// elements at N = 3 28.8 -> 27.3 us.  At N = 4 blocks that start in step crowd each other's
+// neighbours out of the cache (64^3 1712 -> 1741 us, against 25^3 100.4 -> 99.5), so they
+// keep the wait that spreads them; there the stress form is asked for before the
+// thermodynamics instead (64^3 1707, 25^3 99.8; with EARLY it costs 1 % of the N = 3 step).
 template <int Nq, bool DIFF, bool ISO, int MODE, bool WIDE>
 __global__ void __launch_bounds__((block_threads<Nq, WIDE>()))
 __attribute__((amdgpu_waves_per_eu(!WIDE && Nq == 5 ? 6 : 1)))
@@ -531,9 +539,17 @@ k_tendency_mix(KParams P, MixParams MP, AffArrays A, ElemSet ES, const double *_
     if (e < 0) return;
     const int64_t ce = static_class(A, e);
     __shared__ int32_t nb[6];  // the element's face neighbours
-    if (threadIdx.x < 6) nb[threadIdx.x] = A.nbe[6 * e + threadIdx.x];
     const int n = threadIdx.x;
-    if (n < Nq * Nq) sD[n] = (float)A.D[n];
+    constexpr bool EARLY = Nq == 4 && !WIDE;
+    int32_t nbn = 0;
+    double Dn = 0.0;
+    if (EARLY) {
+        nbn = A.nbe[6 * e + min(n, 5)];
+        Dn = A.D[min(n, Nq * Nq - 1)];
+    } else {
+        if (n < 6) nb[n] = A.nbe[6 * e + n];
+        if (n < Nq * Nq) sD[n] = (float)A.D[n];
+    }
     const bool act = n < Np;
     const int i = n % Nq, j = (n / Nq) % Nq, k = n / (Nq * Nq);
     const double *ge = A.geo + (int64_t)AFF_GEO * e;
@@ -567,6 +583,12 @@ k_tendency_mix(KParams P, MixParams MP, AffArrays A, ElemSet ES, const double *_
         const double *qb = Q + (int64_t)Np * 5 * e + n;
 #pragma unroll
         for (int s = 0; s < 5; ++s) q[s] = qb[Np * s];
+        if (DIFF && !EARLY) {
+            const float *gb = gfi + (int64_t)Np * L::NGF * e + n;
+#pragma unroll
+            for (int s = 0; s < L::NREAD; ++s) sf[s] = gb[Np * s];
+        }
+        const double Wn = A.W[n];
         const double *ab = A.sa + (int64_t)Np * P.naux * ce + n;
         if (P.a_Phi >= 0) Phi = ab[(int64_t)Np * P.a_Phi];
         if (P.a_ref_p >= 0) ref_p = ab[(int64_t)Np * P.a_ref_p];
@@ -593,12 +615,12 @@ k_tendency_mix(KParams P, MixParams MP, AffArrays A, ElemSet ES, const double *_
         uf[0] = qf[1] * ri;
         uf[1] = qf[2] * ri;
         uf[2] = qf[3] * ri;
-        if (DIFF) {
+        if (DIFF && EARLY) {
             const float *gb = gfi + (int64_t)Np * L::NGF * e + n;
 #pragma unroll
             for (int s = 0; s < L::NREAD; ++s) sf[s] = gb[Np * s];
         }
-        const double Md = ge[3] * A.W[n];
+        const double Md = ge[3] * Wn;
         MI = (float)recip_d(Md);
         const float M = (float)Md;
 #pragma unroll
@@ -626,6 +648,8 @@ k_tendency_mix(KParams P, MixParams MP, AffArrays A, ElemSet ES, const double *_
             for (int s = 0; s < 5; ++s) sF[ax][s][n] = x * F[s];
         }
     }
+    if (EARLY && n < 6) nb[n] = nbn;
+    if (EARLY && n < Nq * Nq) sD[n] = (float)Dn;
     __syncthreads();
     // volume divergence and gravity source of this node, while sF holds the fluxes
     float T[5];
