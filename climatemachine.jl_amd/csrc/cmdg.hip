@@ -818,7 +818,10 @@ int create_impl(const cmdg_desc *d, const cmdg_brick *brick, void *stream, cmdg_
             // mixed context whose face neighbours would, in storage order, leave one XCD's L2
             // before the gradient pass gathers their state (the 90th percentile of the
             // storage distance between face neighbours, in state bytes, above 4 MiB) walks
-            // 12 x 12 columns spanning y in both passes.
+            // 12 x 12 columns spanning y in both passes.  Where a state is at most 10 MiB (2048
+            // elements at N = 4, 4096 at N = 3) both passes keep the storage order: each then
+            // finds what the pass before wrote in its own XCD's L2 (4 MiB of 32 each), which
+            // passes in different orders do not, and a block reads no list entry.
             // Measured on one box, chosen form (mixed + learned closure):
             //   96^3 (distance 9216 elements, 46 MB): tendency pass in 8^3 tiles 55.0 GDOF/s;
             //     both passes in 8^3 tiles 55.7-56.0 (edge 6 / 12 / 16: 55.3 / 56.2 / 55.8);
@@ -830,6 +833,10 @@ int create_impl(const cmdg_desc *d, const cmdg_brick *brick, void *stream, cmdg_
             // 2338 / 2258, 48^3 977 / 943 / 965, 32^3 297 / 298 / 286, 33^3 347 / 343 / 341,
             // 37 x 52 x 43 743 / 749 / 740, 25^3 131 / 130 / 130.  FP64 gradient: storage
             // order 579 at 48^3, any tile 618-640.
+            // Small meshes, us a call, tendency in tiles / both in storage order: N = 4 mixed
+            // learned 1536 elements 267 / 244, 2048 298 / 282, 3072 420 / 419; FP64 2048 320 /
+            // 303, 3072 476 / 481, 16^3 299 / 311; N = 3 mixed 2048 294 / 266, 3072 339 / 317;
+            // FP64 2048 242 / 209, 4096 313 / 309; N = 3 mixed 7429 620 / 643.
             bool far = false;
             if (d->precision == CMDG_MIXED) {
                 std::vector<int64_t> gap;
@@ -843,7 +850,9 @@ int create_impl(const cmdg_desc *d, const cmdg_brick *brick, void *stream, cmdg_
                     far = (double)*q * Np * 5 * sizeof(double) > 4.0 * 1024 * 1024;
                 }
             }
-            const char *tile_env = std::getenv("CMDG_ELEMENT_TILE");
+            const char *tile_env = std::getenv("CMDG_ELEMENT_TILE"), *penv = std::getenv("CMDG_TILED_PASSES");
+            const bool resident = (double)E * Np * 5 * sizeof(double) <= 10.0 * 1024 * 1024;
+            const std::string passes = penv ? penv : far ? "both" : resident && !tile_env ? "none" : "tendency";
             int T[3] = {8, d->precision == CMDG_MIXED ? 8 : 0, 8};
             if (far) T[0] = 12, T[1] = 0, T[2] = 12;
             if (tile_env && std::strchr(tile_env, ',')) {
@@ -853,10 +862,9 @@ int create_impl(const cmdg_desc *d, const cmdg_brick *brick, void *stream, cmdg_
             }
             std::vector<int32_t> order;
             const int64_t nax[3] = {brick ? brick->ne[0] : 0, brick ? brick->ne[1] : 0, brick ? brick->ne[2] : 0};
-            if (brick ? tiled_order_lattice(lat, nax, E, T, order) : tiled_order(d, Np, T, order)) {
+            if (passes != "none" &&
+                (brick ? tiled_order_lattice(lat, nax, E, T, order) : tiled_order(d, Np, T, order))) {
                 if ((rc = upload(c, &c->d_order, order.data(), order.size()))) return rc;
-                const char *penv = std::getenv("CMDG_TILED_PASSES");
-                const std::string passes = penv ? penv : (far ? "both" : "tendency");
                 if (passes == "both" || passes == "gradient") c->ord_grad = c->d_order;
                 if (passes == "both" || passes == "tendency") c->ord_tend = c->d_order;
             }
@@ -864,10 +872,11 @@ int create_impl(const cmdg_desc *d, const cmdg_brick *brick, void *stream, cmdg_
     }
     // Wide blocks (face tasks in waves of their own, beside the volume waves) where the
     // mesh leaves the chip idle: up to 3 elements a CU at N = 4 and 6 at N = 3, all in
-    // flight at once.  Without / with, us a pass: N = 4 FP64 128 elements 38 / 32 (Euler
-    // step), 162 / 135 (2 LES steps), 512 176 / 158, 768 234 / 226 and 272 / 273, 1024
-    // 214 / 259; mixed 128 142 / 122, 768 203 / 186, 1024 195 / 182 and 107 / 117; N = 3
-    // 1536 225 / 214, 271 / 267, 277 / 251, 2048 243 / 267, 310 / 296.  The general kernels'
+    // flight at once.  Without / with, us a pass: N = 4 FP64 128 elements 38.6 / 31.3 (Euler
+    // step), 162 / 135 (2 LES steps), 512 176 / 158, 768 212 / 199, 1024 215 / 256 and 251 /
+    // 311 with gravity; mixed 128 72.6 / 63.0 (a learned step), 768 192 / 176, 1024 195 / 179
+    // and 107 / 117 with gravity, 1536 245 / 264; N = 3 FP64 1536 193 / 182, 2048 210 / 226,
+    // mixed 236 / 233 and 267 / 267.  The general kernels'
     // line at N = 4 lies a block a CU lower (their tasks hold more registers): 256 170 / 136,
     // 512 214 / 184 and 245 / 229 with gravity, 768 236 / 252 and 285 / 311; N = 3 1536 232 /
     // 214 and 281 / 264, 2744 334 / 332 and 409 / 425.
