@@ -6,12 +6,12 @@
 //
 //   k_gradient   (diffusive models only) gradient argument G(q) staged in LDS,
 //                tensor-product derivative along r/s/t, lifted central face jumps
-//                evaluated by the lanes that own the face nodes, gradient-flux
+//                evaluated as 6 Nfp tasks over the block's lanes, gradient-flux
 //                transform; writes the gradient flux (Np, ngf, nelem).
 //   k_tendency   first + second order flux at each node, contravariant flux
 //                M (xi_a . F) staged in LDS, weak divergence D^T along r/s/t,
-//                gravity source, Rusanov/central face fluxes evaluated by the
-//                lanes owning the face nodes (periodic neighbours come from vmap+
+//                gravity source, Rusanov/central face fluxes evaluated as 6 Nfp
+//                tasks over the block's lanes (periodic neighbours come from vmap+
 //                on the device), and an epilogue that either writes
 //                alpha*RHS + beta*tendency or performs the whole low-storage
 //                Runge-Kutta stage update.
