@@ -414,15 +414,15 @@ bool static_classes(const cmdg_desc *d, const KParams &P, int Np, std::vector<in
 // on the same XCD those lines are still in that XCD's L2.  The storage order of a
 // stacked brick puts the y neighbours a whole x-y row of columns apart (625 elements
 // at 25^3, 9216 at 96^3: tens of MB, far beyond the 4 MB L2), so launches walk the
-// elements in T x T x T tiles instead: z fastest inside a tile, then x, then y, and
-// the tiles in the same order -- every neighbour inside a tile is at most T^2
-// positions away.  The lattice position of each element comes from its centroid
+// elements in tiles or columns instead: z fastest inside one, then x, then y, and
+// the tiles in the same order -- every neighbour inside a tile is at most its x-z
+// cross-section away.  The lattice position of each element comes from its centroid
 // (vgeo x1, x2, x3); returns false, keeping the storage order, when the centroids do
 // not form a complete lattice or the descriptor has no coordinates.
 bool tiled_order_lattice(const std::vector<int64_t> idx[3], const int64_t nax[3], int64_t E, const int T[3],
-                         std::vector<int32_t> &order);
+                         double edge, std::vector<int32_t> &order);
 
-bool tiled_order(const cmdg_desc *d, int Np, const int T[3], std::vector<int32_t> &order) {
+bool tiled_order(const cmdg_desc *d, int Np, const int T[3], double edge, std::vector<int32_t> &order) {
     const int64_t E = d->nelem;
     if (T[0] < 0 || T[1] < 0 || T[2] < 0 || d->nvgeo < 15 || E > INT32_MAX) return false;
     std::vector<int64_t> idx[3];
@@ -449,22 +449,42 @@ bool tiled_order(const cmdg_desc *d, int Np, const int T[3], std::vector<int32_t
             idx[a][e] = it - lev.begin();
         }
     }
-    return tiled_order_lattice(idx, nax, E, T, order);
+    return tiled_order_lattice(idx, nax, E, T, edge, order);
+}
+
+// Columns along x and z (cx, cz) of an nx by nz cross-section: extents near edge, their
+// number a multiple of the 8 XCDs (each then walks whole columns of its own: a column cut
+// between two XCDs is gathered across the cut by both), axes divided exactly if it costs
+// little.  The weights order the choices; any multiple of 8 near the edge does as well.
+void column_counts(int64_t nx, int64_t nz, double edge, int64_t &cx, int64_t &cz) {
+    double best = 1e300;
+    const auto lo = [&](int64_t n) { return std::max<int64_t>(1, (int64_t)((double)n / (2.0 * edge))); };
+    const auto hi = [&](int64_t n) { return std::max<int64_t>(1, std::min<int64_t>(n, (int64_t)(2.0 * (double)n / edge) + 1)); };
+    for (int64_t a = lo(nx); a <= hi(nx); ++a)
+        for (int64_t b = lo(nz); b <= hi(nz); ++b) {
+            const double cost = std::fabs(std::log((double)nx / (edge * (double)a))) +
+                                std::fabs(std::log((double)nz / (edge * (double)b))) + (a * b % 8 ? 1.0 : 0.0) +
+                                (nx % a ? 0.2 : 0.0) + (nz % b ? 0.2 : 0.0);
+            if (cost < best) best = cost, cx = a, cz = b;
+        }
 }
 
 // The tile order of elements at lattice positions idx[a][e] of an nax[0] x nax[1] x
 // nax[2] lattice, tiles of T[0] x T[1] x T[2] elements (0: the whole axis), z fastest
 // then x then y within a tile and between tiles (false when the positions do not fill
-// the lattice once each).
+// the lattice once each).  With an edge > 0 instead of T: columns spanning y, cx by cz of
+// them with extents that differ by at most one, chosen by column_counts.
 bool tiled_order_lattice(const std::vector<int64_t> idx[3], const int64_t nax[3], int64_t E, const int T[3],
-                         std::vector<int32_t> &order) {
+                         double edge, std::vector<int32_t> &order) {
     if (E > INT32_MAX || nax[0] * nax[1] * nax[2] != E) return false;
-    int64_t t[3];
+    int64_t t[3], cnt[3] = {1, 1, 1};
     for (int a = 0; a < 3; ++a) {
         if (T[a] < 0) return false;
         t[a] = T[a] == 0 ? nax[a] : std::min<int64_t>(T[a], nax[a]);
+        cnt[a] = (nax[a] + t[a] - 1) / t[a];
     }
-    const int64_t ntx = (nax[0] + t[0] - 1) / t[0], ntz = (nax[2] + t[2] - 1) / t[2];
+    if (edge > 0.0) column_counts(nax[0], nax[2], edge, cnt[0], cnt[2]), cnt[1] = 1;
+    const auto tile_of = [&](int a, int64_t i) { return edge > 0.0 ? i * cnt[a] / nax[a] : i / t[a]; };
     std::vector<std::pair<int64_t, int32_t>> key(E);
     std::vector<char> seen(E, 0);
     for (int64_t e = 0; e < E; ++e) {
@@ -472,8 +492,8 @@ bool tiled_order_lattice(const std::vector<int64_t> idx[3], const int64_t nax[3]
         const int64_t cell = iz + nax[2] * (ix + nax[0] * iy);
         if (seen[cell]) return false;  // two elements at one lattice point
         seen[cell] = 1;
-        const int64_t tile = iz / t[2] + ntz * (ix / t[0] + ntx * (iy / t[1]));
-        key[e] = {((tile * t[1] + iy % t[1]) * t[0] + ix % t[0]) * t[2] + iz % t[2], (int32_t)e};
+        const int64_t tile = tile_of(2, iz) + cnt[2] * (tile_of(0, ix) + cnt[0] * tile_of(1, iy));
+        key[e] = {tile * E + iz + nax[2] * (ix + nax[0] * iy), (int32_t)e};
     }
     std::sort(key.begin(), key.end());
     order.resize(E);
@@ -813,26 +833,24 @@ int create_impl(const cmdg_desc *d, const cmdg_brick *brick, void *stream, cmdg_
             // tiled traversal.  CMDG_ELEMENT_TILE=T sets cubic tiles of edge T (0 keeps
             // the storage order) and "TX,TY,TZ" tile extents along x, y, z (0: the whole
             // axis); CMDG_TILED_PASSES = tendency, gradient, both or none chooses the passes
-            // that walk the tiles.  Default: an FP64 context's tendency pass walks 8 x 8
-            // columns of elements spanning the whole y axis, a mixed context's 8^3 tiles.  A
+            // that walk the tiles.  Default: the tendency pass walks columns of elements
+            // spanning the whole y axis, about 10 x 10 (column_counts).  A
             // mixed context whose face neighbours would, in storage order, leave one XCD's L2
             // before the gradient pass gathers their state (the 90th percentile of the
             // storage distance between face neighbours, in state bytes, above 4 MiB) walks
-            // 12 x 12 columns spanning y in both passes.  Where a state is at most 10 MiB (2048
+            // them in both passes.  Where a state is at most 10 MiB (2048
             // elements at N = 4, 4096 at N = 3) both passes keep the storage order: each then
             // finds what the pass before wrote in its own XCD's L2 (4 MiB of 32 each), which
             // passes in different orders do not, and a block reads no list entry.
-            // Measured on one box, chosen form (mixed + learned closure):
-            //   96^3 (distance 9216 elements, 46 MB): tendency pass in 8^3 tiles 55.0 GDOF/s;
-            //     both passes in 8^3 tiles 55.7-56.0 (edge 6 / 12 / 16: 55.3 / 56.2 / 55.8);
-            //     both in 12 x 12 columns 56.6 (10 x 10: 56.1, 14 x 14: 55.8, 8 x 8: 56.1);
-            //     mixed + Smagorinsky-Lilly 59.6 / 60.3 / 60.3;
-            //   25^3 (625 elements, 3.1 MB): tendency pass in 8^3 tiles 50.0-50.3; both
-            //     passes 49.3; 12 x 12 columns 49.2 (tendency pass), 48.6 (both).
-            // FP64 tendency, us a launch in 8^3 tiles / 6 x 6 / 8 x 8 columns: 64^3 2299 /
-            // 2338 / 2258, 48^3 977 / 943 / 965, 32^3 297 / 298 / 286, 33^3 347 / 343 / 341,
-            // 37 x 52 x 43 743 / 749 / 740, 25^3 131 / 130 / 130.  FP64 gradient: storage
-            // order 579 at 48^3, any tile 618-640.
+            // us a call, 8^3 tiles (mixed, 12 x 12 columns where far; FP64 8 x 8) with their
+            // remainders / columns in a multiple of 8 near edge 8 / 10 / 12: mixed 20^3 882 /
+            // 853 / 862 / 862, 25^3 831 / 825 / 808 / 816, 32^3 3520 / 3325 / 3325 / 3381, 40^3
+            // 6957 / 6668 / 6668 / 6668, 56^3 18940 / 18580 / 18600 / 18510, 64^3 28220 / 27230
+            // / 27220 / 27900, 96^3 already had 8 x 8 columns of 12 x 12; FP64 25^3 2448 / 2445 /
+            // 2408 / 2453, 48^3 14770 / 14735 / 14607 / 14617, 37 x 52 x 43 11160 / 11020 /
+            // 11000 / 11010; N = 3 mixed 621 / 616 / 615 / 633.  A count that is no multiple of 8
+            // gives most of it away (33^3 mixed in 3 x 3 2000, in 4 x 4 1954).
+            // FP64 gradient: storage order 579 us a launch at 48^3, any tile 618-640.
             // Small meshes, us a call, tendency in tiles / both in storage order: N = 4 mixed
             // learned 1536 elements 267 / 244, 2048 298 / 282, 3072 420 / 419; FP64 2048 320 /
             // 303, 3072 476 / 481, 16^3 299 / 311; N = 3 mixed 2048 294 / 266, 3072 339 / 317;
@@ -853,8 +871,8 @@ int create_impl(const cmdg_desc *d, const cmdg_brick *brick, void *stream, cmdg_
             const char *tile_env = std::getenv("CMDG_ELEMENT_TILE"), *penv = std::getenv("CMDG_TILED_PASSES");
             const bool resident = (double)E * Np * 5 * sizeof(double) <= 10.0 * 1024 * 1024;
             const std::string passes = penv ? penv : far ? "both" : resident && !tile_env ? "none" : "tendency";
-            int T[3] = {8, d->precision == CMDG_MIXED ? 8 : 0, 8};
-            if (far) T[0] = 12, T[1] = 0, T[2] = 12;
+            const double edge = tile_env ? 0.0 : 10.0;
+            int T[3] = {0, 0, 0};
             if (tile_env && std::strchr(tile_env, ',')) {
                 if (std::sscanf(tile_env, "%d,%d,%d", &T[0], &T[1], &T[2]) != 3) T[0] = T[1] = T[2] = -1;
             } else if (tile_env) {
@@ -863,7 +881,7 @@ int create_impl(const cmdg_desc *d, const cmdg_brick *brick, void *stream, cmdg_
             std::vector<int32_t> order;
             const int64_t nax[3] = {brick ? brick->ne[0] : 0, brick ? brick->ne[1] : 0, brick ? brick->ne[2] : 0};
             if (passes != "none" &&
-                (brick ? tiled_order_lattice(lat, nax, E, T, order) : tiled_order(d, Np, T, order))) {
+                (brick ? tiled_order_lattice(lat, nax, E, T, edge, order) : tiled_order(d, Np, T, edge, order))) {
                 if ((rc = upload(c, &c->d_order, order.data(), order.size()))) return rc;
                 if (passes == "both" || passes == "gradient") c->ord_grad = c->d_order;
                 if (passes == "both" || passes == "tendency") c->ord_tend = c->d_order;

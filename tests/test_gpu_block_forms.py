@@ -83,3 +83,17 @@ def test_wide_blocks_general(name, N, steps):
     env = {"CMDG_GENERAL_GEOMETRY": "1"}
     _same(_run(*case, abi.FP64, steps, CMDG_WIDE_BLOCKS="0", **env),
           _run(*case, abi.FP64, steps, CMDG_WIDE_BLOCKS="1", **env))
+
+
+@pytest.mark.parametrize("shape", [(11, 3, 23), (2, 5, 37), (21, 2, 20)])
+@pytest.mark.parametrize("precision", [abi.FP64, abi.MIXED])
+def test_columns_walk_every_element(precision, shape):
+    """The default columns on cross-sections that no column count divides."""
+    from cmdg.grid import uniform_brick
+    prm = atmos.ideal_gas_parameters()
+    grid = uniform_brick(shape, (0.0, 0.0, 0.0), (6.0, 5.0, 4.0), N=3)
+    cfg = atmos.AtmosConfig(prm, turbulence=abi.SMAGORINSKY_LILLY, C_smag=0.21)
+    Q0 = atmos.taylor_green(prm, grid, mach=0.1)
+    Q0[:, 1:4, :] *= 1 + 0.05 * np.random.default_rng(7).uniform(-1, 1, Q0[:, 1:4, :].shape)
+    case = (cfg, grid, atmos.init_aux(cfg, grid), Q0)
+    _same(_run(*case, precision, 0, CMDG_TILED_PASSES="both"), _run(*case, precision, 0, CMDG_ELEMENT_TILE="0"))
