@@ -889,8 +889,9 @@ int create_impl(const cmdg_desc *d, const cmdg_brick *brick, void *stream, cmdg_
         }
     }
     // Wide blocks (face tasks in waves of their own, beside the volume waves) where the
-    // mesh leaves the chip idle: up to 3 elements a CU at N = 4 and 6 at N = 3, all in
-    // flight at once.  Without / with, us a pass: N = 4 FP64 128 elements 38.6 / 31.3 (Euler
+    // mesh leaves the chip idle: up to 3 elements a CU at N = 4 (5 mixed without gravity, whose
+    // kernels hold the fewest registers: 1280 elements 223 / 212, Smagorinsky-Lilly 193 / 182,
+    // Euler 55.7 / 52.8) and 6 at N = 3, all in flight at once.  Without / with, us a pass: N = 4 FP64 128 elements 38.6 / 31.3 (Euler
     // step), 162 / 135 (2 LES steps), 512 176 / 158, 768 212 / 199, 1024 215 / 256 and 251 /
     // 311 with gravity; mixed 128 72.6 / 63.0 (a learned step), 768 192 / 176, 1024 195 / 179
     // and 107 / 117 with gravity, 1536 245 / 264; N = 3 FP64 1536 193 / 182, 2048 210 / 226,
@@ -900,7 +901,8 @@ int create_impl(const cmdg_desc *d, const cmdg_brick *brick, void *stream, cmdg_
     // 214 and 281 / 264, 2744 334 / 332 and 409 / 425.
     // (CMDG_WIDE_BLOCKS=0 or 1 chooses.)
     const char *wenv = std::getenv("CMDG_WIDE_BLOCKS");
-    c->wide = wenv ? wenv[0] == '1' : E <= (Nq != 5 ? 1536 : c->affine ? 768 : 512);
+    const bool light = d->precision == CMDG_MIXED && P.a_gPhi < 0;
+    c->wide = wenv ? wenv[0] == '1' : E <= (Nq != 5 ? 1536 : light ? 1280 : c->affine ? 768 : 512);
     if (!c->affine) {
         // general meshes: per-node geometry xi (9), M, MI, the face geometry and the
         // neighbour node of every face node (affine bricks read none of these)
