@@ -274,13 +274,15 @@ __global__ void __launch_bounds__(128) k_element_average_pqr(float *__restrict__
 constexpr int MP_W1 = 0, MP_B1 = 320, MP_W2 = 352, MP_B2 = 1376, MP_W3 = 1408, MP_B3 = 1440, MLP_NPARAM = 1441;
 constexpr int GRAD_W = MLP_NPARAM + 1;  // + loss
 // A row of partial gradients is one workgroup's.  The caller's workspace holds a row for
-// every TRAIN_TB samples; a large batch fills TRAIN_ROWS of them, one a CU, and its waves take several
-// tiles each.
-constexpr int TRAIN_TB = 64, TRAIN_ROWS = 256;
+// every TRAIN_TB samples; a batch above 16384 fills TRAIN_ROWS of them, one a CU, whose waves
+// take several tiles each, until a row holds ROW_SAMPLES samples (a batch of 65536), and from
+// there on a row for every ROW_SAMPLES: what is summed in FP32 before the rows' FP64 sum does
+// not grow with the batch.
+constexpr int TRAIN_TB = 64, TRAIN_ROWS = 256, ROW_SAMPLES = 256;
 constexpr int TRAIN_NT = 256, TRAIN_TILE = 16;  // threads a workgroup; samples a wave's tile
 inline int64_t train_rows(int64_t batch) {
-    const int64_t nb = (batch + TRAIN_TB - 1) / TRAIN_TB;
-    return nb < TRAIN_ROWS ? nb : TRAIN_ROWS;
+    const int64_t nb = (batch + TRAIN_TB - 1) / TRAIN_TB, full = (batch + ROW_SAMPLES - 1) / ROW_SAMPLES;
+    return nb < TRAIN_ROWS ? nb : full < TRAIN_ROWS ? TRAIN_ROWS : full;
 }
 
 __device__ __forceinline__ float silu_fwd(float a, float &dsilu) {
@@ -307,7 +309,9 @@ __device__ __forceinline__ float silu_fwd(float a, float &dsilu) {
 // 170 registers ran one wave a SIMD, its weight-gradient loops 64 serial LDS reads long).
 // What is left is the gather (13 words of a sample lie in 13 lines): rows in order take 15.
 // 256 rows of partials, one workgroup a CU, are faster than 512 or 1024 from 32768 samples on
-// (27 against 31 and 33 us for the two launches at 65536), and equal below.
+// (27 against 31 and 33 us for the two launches at 65536), and equal below.  Above 65536 a row
+// keeps to 256 samples: 268 us at 2^20, 1016 at 2^22, where 256 rows of any length took 250 and
+// 949 but summed up to 16384 samples a row in FP32 (one repeated tile of samples: 4e-5 off).
 __global__ void __launch_bounds__(TRAIN_NT)
 k_mlp_grad(const float *__restrict__ params, const float *__restrict__ shift, const float *__restrict__ scale,
            const float *__restrict__ samples, int64_t ld, const int64_t *__restrict__ idx, int64_t batch,
