@@ -739,14 +739,6 @@ int create_impl(const cmdg_desc *d, const cmdg_brick *brick, void *stream, cmdg_
     if (d->precision != CMDG_MIXED && (rc = upload<double>(c, &c->d_gf, nullptr, (size_t)Np * c->ngf * E)))
         return rc;
     if ((rc = upload<double>(c, &c->d_Qs, nullptr, (size_t)Np * 5 * E))) return rc;
-    // a third state buffer for odd step counts (cmdg_lsrk54_steps), up to 1 GiB and where
-    // there is room (CMDG_THIRD_STATE_BUFFER=0: never): without it such a call copies the state
-    const char *qenv = std::getenv("CMDG_THIRD_STATE_BUFFER");
-    if (!(qenv && qenv[0] == '0') && (size_t)Np * 5 * E * sizeof(double) <= (size_t)1 << 30 &&
-        hipMalloc((void **)&c->d_Qt, (size_t)Np * 5 * E * sizeof(double)) != hipSuccess) {
-        c->d_Qt = nullptr;
-        (void)hipGetLastError();
-    }
     if (c->d_gf &&
         (rc = check_hip(c, hipMemset(c->d_gf, 0, (size_t)Np * c->ngf * E * sizeof(double)), "hipMemset")))
         return rc;
@@ -963,6 +955,19 @@ int create_impl(const cmdg_desc *d, const cmdg_brick *brick, void *stream, cmdg_
             c->AA.gphi32 = c->d_gphi32;
         }
         if (c->learned && (rc = upload<MlpDev>(c, &c->d_mlp, nullptr, 1))) return rc;
+    }
+    // Last, what the context can do without: a third state buffer for odd step counts
+    // (cmdg_lsrk54_steps), for a state of at most 1 GiB and a 64th of the memory still free, so
+    // that it is never what a later allocation misses on a card that is in use
+    // (CMDG_THIRD_STATE_BUFFER=0: never).  Without it such a call copies the state.
+    const char *qenv = std::getenv("CMDG_THIRD_STATE_BUFFER");
+    const size_t state_bytes = (size_t)Np * 5 * E * sizeof(double);
+    size_t free_bytes = 0, total_bytes = 0;
+    if (!(qenv && qenv[0] == '0') && state_bytes <= (size_t)1 << 30 &&
+        (hipMemGetInfo(&free_bytes, &total_bytes) != hipSuccess || state_bytes > free_bytes / 64 ||
+         hipMalloc((void **)&c->d_Qt, state_bytes) != hipSuccess)) {
+        c->d_Qt = nullptr;
+        (void)hipGetLastError();
     }
     return CMDG_OK;
 }

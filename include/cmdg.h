@@ -110,7 +110,9 @@ typedef struct cmdg_ctx cmdg_ctx;
 /* Build a DG context (the DGModel of src/Numerics/DGMethods/DGModel.jl:22-65):
  * copies geometry/connectivity to the device, takes ownership of a device copy of
  * the auxiliary state (DGModel.state_auxiliary) and allocates scratch (gradient
- * flux, ping-pong state).  `stream` is a hipStream_t (NULL = default stream). */
+ * flux, ping-pong state; last, for a state of at most 1 GiB and a 64th of the device
+ * memory then free, a third state buffer that saves a copy in calls of an odd number of
+ * steps).  `stream` is a hipStream_t (NULL = default stream). */
 int cmdg_create(const cmdg_desc *desc, void *stream, cmdg_ctx **out);
 
 /* An axis-aligned brick of ne[0] x ne[1] x ne[2] elements with break points x[a]
