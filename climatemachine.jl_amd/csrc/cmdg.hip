@@ -168,8 +168,7 @@ template <class T> int upload(cmdg_ctx *c, T **dst, const T *src, size_t count) 
 // ES: the elements of this launch (affine kernels; the general ones take them all).
 template <int Nq>
 int launch_gradient_impl(cmdg_ctx *c, const double *Q, double *Qcopy, int write_aux, const ElemSet &ES) {
-    constexpr int NT = threads_for<Nq>();
-    dim3 grid((unsigned)xcd_grid(c->affine ? ES.count : c->nelem)), block(NT);
+    const dim3 grid((unsigned)xcd_grid(c->affine ? ES.count : c->nelem));
     TimedLaunch tl(c, KIND_GRADIENT);
     // N^2 (Smagorinsky-Lilly) needs theta_v only under a gravitational potential
     const bool buoy = c->P.a_gPhi >= 0;
@@ -229,8 +228,7 @@ int launch_gradient_impl(cmdg_ctx *c, const double *Q, double *Qcopy, int write_
 template <int Nq>
 int launch_tendency_impl(cmdg_ctx *c, const double *Q, double *tend, double alpha, double beta, int mode,
                          double *Qout, double rka, double bdt, int write_aux, int dq_store, const ElemSet &ES) {
-    constexpr int NT = threads_for<Nq>();
-    dim3 grid((unsigned)xcd_grid(c->affine ? ES.count : c->nelem)), block(NT);
+    const dim3 grid((unsigned)xcd_grid(c->affine ? ES.count : c->nelem));
     TimedLaunch tl(c, KIND_TENDENCY);
 #define CMDG_TEND_MIX(DIFF, ISO, MODE)                                                                           \
     do {                                                                                                          \

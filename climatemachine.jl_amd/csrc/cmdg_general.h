@@ -191,7 +191,7 @@ k_gradient(KParams P, KArrays A, const double *__restrict__ Q, double *__restric
 
 // ------------------------------------------------------------------ tendency kernel
 // One side of a face or one node: its fluxes from the state, static fields and gradient flux.
-template <int Nq, bool DIFF, bool SMAG>
+template <int Nq, bool SMAG>
 __device__ __forceinline__ void node_flux2(const KParams &P, const double *__restrict__ gfi,
                                            const double *__restrict__ nui, int nnu, int64_t e, int n,
                                            const double q[5], double F2[3][5]) {
@@ -240,8 +240,8 @@ __device__ __forceinline__ void face_flux(const KParams &P, const KArrays &A, co
     double f2[5];
     if (DIFF && !wall) {
         double Fm[3][5], Fp[3][5];
-        node_flux2<Nq, DIFF, SMAG>(P, gfi, nui, nnu, e, vn, q, Fm);
-        node_flux2<Nq, DIFF, SMAG>(P, gfi, nui, nnu, ep, vp, qp, Fp);
+        node_flux2<Nq, SMAG>(P, gfi, nui, nnu, e, vn, q, Fm);
+        node_flux2<Nq, SMAG>(P, gfi, nui, nnu, ep, vp, qp, Fp);
 #pragma unroll
         for (int s = 0; s < 5; ++s)
             f2[s] = ((Fm[0][s] + Fp[0][s]) * h[0] + (Fm[1][s] + Fp[1][s]) * h[1]) + (Fm[2][s] + Fp[2][s]) * h[2];
@@ -316,7 +316,7 @@ k_tendency(KParams P, KArrays A, const double *__restrict__ Q, const double *__r
         flux1(P, q, t.p, a.ref_p, F);
         if (DIFF) {
             double F2[3][5];
-            node_flux2<Nq, DIFF, SMAG>(P, gfi, nui, nnu, e, n, q, F2);
+            node_flux2<Nq, SMAG>(P, gfi, nui, nnu, e, n, q, F2);
 #pragma unroll
             for (int d = 0; d < 3; ++d)
 #pragma unroll
