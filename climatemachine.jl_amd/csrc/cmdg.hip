@@ -451,9 +451,14 @@ bool tiled_order(const cmdg_desc *d, int Np, const int T[3], double edge, std::v
 }
 
 // Columns along x and z (cx, cz) of an nx by nz cross-section: extents near edge, their
-// number a multiple of the 8 XCDs (each then walks whole columns of its own: a column cut
-// between two XCDs is gathered across the cut by both), axes divided exactly if it costs
-// little.  The weights order the choices; any multiple of 8 near the edge does as well.
+// number a multiple of the 8 XCDs where one lies near it (each then walks whole columns of its
+// own, up to the difference of their extents: a column cut between two XCDs is gathered across
+// the cut by both), axes divided exactly if it costs little.  The weights order the choices; any
+// multiple of 8 near the edge does as well.
+// A cross-section with a side of 14 elements or fewer may get fewer columns or another number
+// (13 x 13 one, 30 x 4 three): eight narrow ones gain on some and lose on others.  Speed of
+// two-step calls in eight against the choice: FP64 with gravity 14^3 1.022, 13^3 1.014, without
+// 12 x 40 x 12 1.01, 9 x 60 x 9 0.98; mixed 14^3 0.99, 13^3 0.96, 12 x 40 x 12 1.02, 9 x 60 x 9 0.98.
 void column_counts(int64_t nx, int64_t nz, double edge, int64_t &cx, int64_t &cz) {
     double best = 1e300;
     const auto lo = [&](int64_t n) { return std::max<int64_t>(1, (int64_t)((double)n / (2.0 * edge))); };
@@ -838,8 +843,8 @@ int create_impl(const cmdg_desc *d, const cmdg_brick *brick, void *stream, cmdg_
             // 6957 / 6668 / 6668 / 6668, 56^3 18940 / 18580 / 18600 / 18510, 64^3 28220 / 27230
             // / 27220 / 27900, 96^3 already had 8 x 8 columns of 12 x 12; FP64 25^3 2448 / 2445 /
             // 2408 / 2453, 48^3 14770 / 14735 / 14607 / 14617, 37 x 52 x 43 11160 / 11020 /
-            // 11000 / 11010; N = 3 mixed 621 / 616 / 615 / 633.  A count that is no multiple of 8
-            // gives most of it away (33^3 mixed in 3 x 3 2000, in 4 x 4 1954).
+            // 11000 / 11010; N = 3 mixed 621 / 616 / 615 / 633.  On these a count that is no
+            // multiple of 8 gives most of it away (33^3 mixed in 3 x 3 2000, in 4 x 4 1954).
             // FP64 gradient: storage order 579 us a launch at 48^3, any tile 618-640.
             // Small meshes, us a call, tendency in tiles / both in storage order: N = 4 mixed
             // learned 1536 elements 267 / 244, 2048 298 / 282, 3072 420 / 419; FP64 2048 320 /

@@ -205,8 +205,10 @@ constexpr int viscosity_planes(bool smag, bool buoy) { return smag ? (buoy ? 3 :
 // round trips a block.  In the tendency, likewise, every field of the node is asked for before
 // anything is waited for.  us, gradient + tendency: 48^3 Smagorinsky-Lilly 582 + 972 -> 554 +
 // 955, 33^3 constant viscosity 196 + 341 -> 183 + 334, 25^3 with gravity 107.8 + 147.9 ->
-// 104.5 + 146.5.  The face waves of a wide block read their own neighbour and fill the time
-// (128 elements the same or 1 us a step slower so), so there the matrix stays under its branch.
+// 104.5 + 146.5.  Now, traced over warm calls: 555 + 937, 180 + 324, 105.6 + 143.0; the gradient
+// moves 189 B a node at 48^3, 4.7 TB/s.  The face waves of a wide block read their own
+// neighbour and fill the time (128 elements the same or 1 us a step slower so), so there the
+// matrix stays under its branch.
 template <int Nq, bool SMAG, bool BUOY, bool WIDE>
 __global__ void __launch_bounds__((block_threads<Nq, WIDE>()))
 k_gradient_aff(KParams P, AffArrays A, ElemSet ES, const double *__restrict__ Q, double *__restrict__ aux,
@@ -447,15 +449,15 @@ __device__ __forceinline__ void face_flux_aff(const KParams &P, const AffArrays 
 //   not read; dq_store = 0 leaves the scaled dQ unstored (this stage's rka is 0 and the
 //   next stage is launched with beta = 0).
 // NNU: viscosity planes of nui (Smagorinsky-Lilly; 0: a constant viscosity).
-// What bounds it: nothing alone.  At 48^3 (Smagorinsky-Lilly) the lines that miss L2 are 290 B
-// a node read and 79 written, 5.1 TB/s; VALU issues in 45 % of the cycles, LDS in 27 %; each
-// wave waits two thirds of its life, so waves are what helps.  The horizontal fluxes share
+// What bounds it: nothing alone.  At 48^3 (Smagorinsky-Lilly) the lines that miss L2 are 319 B
+// a node read and 80 written, 5.9 TB/s; VALU issues in 48 % of the cycles, LDS in 29 %; each
+// wave waits 63 % of its life, so waves are what helps.  The horizontal fluxes share
 // one LDS space with the vertical ones and the staged state that follow them, and a face
 // node's own row shares its slot with the flux (16.2 KB a block; three directions at once
 // took 20.0), which with the second-order part of a face taken first (94 registers, 110-122
 // before) lets 5 waves a SIMD run instead of 4.  48^3: 1017 -> 965 us a launch, 33^3 constant
-// viscosity 366 -> 341, 25^3 with gravity 150.5 -> 147.5.  Fewer blocks a CU (LDS padding, 4
-// waves): 8 / 7 / 6 / 5 give 1010 / 1065 / 1150 / 1475 us; nine spilled registers 1332.  Face
+// viscosity 366 -> 341, 25^3 with gravity 150.5 -> 147.5 (now, with what the gradient pass's note
+// adds, 937, 324 and 143).  Fewer blocks a CU (LDS padding, 4 waves): 8 / 7 / 6 / 5 give 1010 / 1065 / 1150 / 1475 us; nine spilled registers 1332.  Face
 // tasks first, both sides read from memory instead of LDS, cut the missed lines to 213 B and
 // cost 1069 us: the added vector-memory instructions weigh more.
 // At Nq = 4 five waves spill.

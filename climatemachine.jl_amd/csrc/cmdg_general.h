@@ -14,7 +14,11 @@
 // 312 -> 138 + 261 (a task's theta_v costs what the faces' order gave), 14^3 27.8 + 52.6 ->
 // 22.8 + 42.7, N = 3 24^3 69 + 132 -> 58 + 102.  A neighbour index read one task ahead
 // lengthens the registers' lives by more than it hides (14 x 12 x 10 viscous right-hand side
-// 35.7 against 36.9 us with it).
+// 35.7 against 36.9 us with it).  A task reads its own side from memory again; with nothing in
+// cache (1 GiB written between calls) the right-hand side gains as much: 14 x 12 x 10 viscous
+// 52.0 -> 48.6 us, 22^3 264 -> 246, Smagorinsky-Lilly 336 -> 263, with gravity 364 -> 325.  Of the
+// meshes timed one lost, warm and cold: N = 3 18^3 viscous 59.0 -> 60.1 (5832 blocks are 1.6
+// rounds of the 14 a CU that LDS lets run; 12^3 24.8 -> 23.3, 22^3 105.6 -> 101.7).
 #pragma once
 #include "cmdg_affine.h"
 

@@ -85,11 +85,11 @@ struct FilterProj {
     double p[2][5][5];
 };
 
-// One axis at a time (11 fields x 770 products a node instead of 11 x 1000 x 2): along x the
-// two children of a pair into X, along y two pairs into Y, along z two halves into the
-// result, each partial sum in registers and passed on through LDS, a row of Nq nodes padded
+// One axis at a time (70 products a node and field, 8 x 5 + 4 x 5 + 2 x 5, instead of
+// 8 x 125): along x the two children of a pair into X, along y two pairs into Y, along z two
+// halves into the result, each partial sum in registers and passed on through LDS, a row of Nq nodes padded
 // to an even number so that two are read at once.  The children of the next pair are loaded
-// while this one is contracted.  48^3 fine elements: 2420 -> 214 us (705 MB, 148 us at the
+// while this one is contracted.  48^3 fine elements: 2176 -> 199 us traced warm (705 MB, 148 us at the
 // copy rate); the sums are shorter, and closer to 64-bit exact, than the triple loop's.
 template <int Nq>
 __global__ void __launch_bounds__(threads_for<Nq>())
@@ -305,7 +305,7 @@ __device__ __forceinline__ float silu_fwd(float a, float &dsilu) {
 // the lanes already hold in register (m, r); only the weights are laid out to match.  The
 // weight gradients contract over samples, for which each matrix is transposed once through
 // the wave's LDS.  b1 rides along as the weight of an eleventh input that is 1.
-// 65536 rows of a 2^21-sample table: 188 -> 23 us (one lane a sample with its activations in
+// 65536 rows of a 2^21-sample table: 187 -> 25 us traced warm (one lane a sample with its activations in
 // 170 registers ran one wave a SIMD, its weight-gradient loops 64 serial LDS reads long).
 // What is left is the gather (13 words of a sample lie in 13 lines): rows in order take 15.
 // 256 rows of partials, one workgroup a CU, are faster than 512 or 1024 from 32768 samples on
@@ -565,7 +565,7 @@ struct InterpMat {
 // its points over p^3) the workgroups walk them with x fastest, as a stacked brick stores them
 // (z fastest, then x, then y), so that one XCD's L2 completes the lines of out, of which an
 // element writes p words; any order is right, the position comes from eijk.
-// 40^3 elements, p = 4: 206 -> 80 us (354 MB, 74 us at the copy rate); with p at run time
+// 40^3 elements, p = 4: 177 -> 77 us traced warm (354 MB, 74 us at the copy rate); with p at run time
 // the index arithmetic held it at 141.
 constexpr int interp_threads(int p) { return p <= 3 ? 64 : p <= 5 ? 128 : 256; }
 template <int Nq, int p>

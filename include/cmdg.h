@@ -321,9 +321,9 @@ int cmdg_not_finite_fields(cmdg_ctx *ctx, const double *Q, int32_t *mask);
  * lattice tiles (z fastest, then x, then y, within and between tiles) so that a
  * block's face neighbours ran shortly before it on the same XCD: by default the
  * tendency pass, in element columns spanning y (about 10 x 10, their number a multiple of
- * the 8 XCDs), and a mixed context whose face neighbours lie farther apart in storage order
- * than one XCD's L2 holds walks them in both passes (a state of at most 10 MiB is walked
- * in storage order: bit 3 clear).
+ * the 8 XCDs unless the cross-section is narrow), and a mixed context whose face
+ * neighbours lie farther apart in storage order than one XCD's L2 holds walks them in both
+ * passes (a state of at most 10 MiB is walked in storage order: bit 3 clear).
  * Setting CMDG_GENERAL_GEOMETRY=1 in the environment before cmdg_create clears bit 0;
  * CMDG_NEIGHBOUR_STATIC_TRACE=1 clears bit 1; CMDG_STATIC_AUX_CLASSES=0 clears bit 2;
  * CMDG_ELEMENT_TILE=T sets cubic tiles of edge T (T = 0 clears bit 3) and
